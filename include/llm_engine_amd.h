@@ -150,7 +150,10 @@ typedef struct le_plan_config {
   int32_t q_heads, kv_heads, head_dim, block_size;
   int32_t kv_dtype;            /* le_dtype of the cache the plan will be run against */
   int32_t partition_tokens;    /* split-K partition of decode rows; 0 = default */
-  int32_t chunk_q_tile;        /* query rows per chunk tile (16 or 32); 0 = default (32) */
+  int32_t chunk_q_tile;        /* query rows per chunk tile (16 or 32); 0 (or less) = default: 32
+                                  with an fp32 cache, else tiles of 128 or 256 query columns
+                                  (row, head), sized and partitioned by the step; a packed plan's
+                                  cfg then holds 0 or -1 here and 0 below */
   int32_t chunk_partition_tokens; /* key partition of chunk tiles; 0 = default */
   int32_t flags;               /* LE_PLAN_* bits below; 0 = the defaults */
   int32_t table_capacity;      /* 0: tables packed exactly. > 0: a fixed layout for a step of
@@ -225,7 +228,7 @@ static inline const int32_t* le_plan_dev_array(const le_step_plan* plan, int64_t
  * (3)(4) Ragged paged attention over a packed step.
  * Decode rows (slices of length 1) run the bandwidth kernel: one workgroup per
  * (row, kv head, context partition), each K/V row read once for the whole
- * GQA group. Prefill-chunk rows run the MFMA tile kernel (bf16 / fp16 tiles
+ * GQA group. Prefill-chunk rows run the MFMA tile kernels (bf16 / fp16 tiles
  * for 16-bit caches, fp32 tiles for an fp32 cache), with a causal mask by
  * absolute position against the cached prefix. Split rows are merged inside
  * their launch. The result equals le_attention_decode on the same step.

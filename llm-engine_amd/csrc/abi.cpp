@@ -273,6 +273,12 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
   // A mixed step is one launch (chunk and decode workgroups in one grid);
   // LE_PLAN_TWO_LAUNCHES runs the two kernels one after the other instead.
   const bool two_launches = (cfg.flags & LE_PLAN_TWO_LAUNCHES) != 0;
+  if (cfg.chunk_q_tile <= 0) {  // chunk items are prefill tiles
+    const bool wide = cfg.chunk_q_tile == le::kWidePrefillTiles;
+    return hip_status(plan->n_decode_items > 0
+                          ? le::attention_ragged_prefill(d, c, wide, act_dtype, kv_dtype, stream)
+                          : le::attention_prefill(c, wide, act_dtype, kv_dtype, stream));
+  }
   if (plan->n_decode_items > 0 && !two_launches)
     return hip_status(le::attention_ragged(d, c, act_dtype, kv_dtype, stream));
   e = le::attention_decode(d, act_dtype, kv_dtype, stream);

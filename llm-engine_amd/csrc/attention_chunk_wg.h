@@ -8,7 +8,10 @@
 // (cpu_model.cpp:144-158 writes every token's K/V before attention runs).
 // The reference has no prefill kernel (attention_prefill.cu:1 is a stub) and
 // runs chunk rows through the decode kernel, re-reading the history once per
-// row; here 32 consecutive rows share every K/V read.
+// row; here 32 consecutive rows share every K/V read. With a 16-bit cache
+// these tiles run where a plan names their row tile or partition, asks for two
+// launches, or has more rows than arrival counters; the prefill tiles
+// (attention_prefill_wg.h) run everywhere else.
 //
 // gfx950 design:
 //   * one 512-thread workgroup (8 waves) per (32-row tile, kv head, key
@@ -149,7 +152,7 @@ template <typename KV, int HD> struct ChunkSmem {
 // itself, kMJ partitions per round of loads: the partition's (m, l) for the
 // row and head, and its normalised output (fp32), requested together, then
 // folded in partition order into a running (max, sum) with rescaling. With at
-// most kMJ partitions the whole merge is one memory round trip, with no LDS
+// most kMJ partitions a round is one memory round trip, with no LDS
 // phase or barrier.
 // Split tiles of a bf16 cache carry their partials as fp16: the tile already
 // rounds its softmax weights to bf16 (2^-9), and a normalised partial is a
@@ -161,21 +164,20 @@ template <typename KV, int HD> struct ChunkSmem {
 // fp16 and fp32 caches keep fp32 partials.
 template <typename KV> constexpr bool kHalfPartials = std::is_same_v<KV, bf16_t>;
 
-template <typename ACT, int HD, int kMJ, bool kHalf>
+template <typename ACT, int HD, int kMJ, bool kHalf, int NTHR = kThreads, int kMG = 2>
 __device__ __forceinline__ void merge_tile(const ChunkParams& p, const ChunkItem& it, __amdgpu_buffer_rsrc_t acc_rsrc,
                                            float* ml, int64_t rec_tile, int base, int J, int G, int kvh, int nq,
                                            int tok0) {
-  constexpr int kMG = 2;  // output 8-vectors per thread and round
   const int tid = threadIdx.x;
   const int per_row = G * (HD / 8);
   const int n_out = nq * per_row;
-  for (int o0 = tid; o0 < n_out; o0 += kMG * kThreads) {
+  for (int o0 = tid; o0 < n_out; o0 += kMG * NTHR) {
     int64_t rec_base[kMG];
     int d8[kMG];
     float M[kMG], L[kMG], sum[kMG][8];
 #pragma unroll
     for (int gi = 0; gi < kMG; gi++) {
-      const int o = min(o0 + gi * kThreads, n_out - 1);
+      const int o = min(o0 + gi * NTHR, n_out - 1);
       const int r = o / per_row, rem = o - r * per_row;
       const int g = rem / (HD / 8);
       d8[gi] = rem - g * (HD / 8);
@@ -231,7 +233,7 @@ __device__ __forceinline__ void merge_tile(const ChunkParams& p, const ChunkItem
     }
 #pragma unroll
     for (int gi = 0; gi < kMG; gi++) {
-      const int o = o0 + gi * kThreads;
+      const int o = o0 + gi * NTHR;
       if (o < n_out) {
         const int r = o / per_row, rem = o - r * per_row;
         const int g = rem / (HD / 8);

@@ -17,6 +17,7 @@
 // workgroups run as eight waves as well. The LDS is the larger of the two.
 #include "attention_chunk_wg.h"
 #include "attention_decode_wg.h"
+#include "attention_prefill_wg.h"
 
 namespace le {
 namespace {
@@ -47,8 +48,52 @@ __global__ __launch_bounds__(kRaggedThreads) void ragged_kernel(DecodeParams dp,
   }
 }
 
+// The same for chunk rows cut into prefill tiles (16-bit caches): 256-thread
+// workgroups of both kinds, two of any per CU. Bound like the prefill kernel
+// in steps with large chunks, by the decode rows' streaming and the tiles'
+// serial chain in small ones. Against the kernel above (us per call): 2 x 512
+// rows after 1024 keys and 32 decode rows of 256-2048, 14/2 heads x 64, 28.9
+// and 25.6; 8 x 512 after 4096, 32/4 x 64, 369 and 171; one chunk of 64 after
+// nothing, 16.2 and 11.6; 8/8 x 128 and 8 x 512 after 1024, 321 and 80.
+template <typename KV, int HD> union RaggedPrefillSmem {
+  pre::PrefillSmem<HD> c;
+  dec::DecodeSmem<KV, HD, pre::kWaves> d;
+};
+
+template <typename ACT, typename KV, int HD, int NC>
+__global__ __launch_bounds__(pre::kThreads, 2) void ragged_prefill_kernel(DecodeParams dp, ChunkParams cp) {
+  __shared__ RaggedPrefillSmem<KV, HD> sm;
+  const int n_chunk_wg = cp.n_items * cp.kv_heads;
+  const int b = blockIdx.x;
+  if (b < n_chunk_wg) {
+    pre::prefill_wg<ACT, KV, HD, NC>(cp, sm.c, b / cp.kv_heads, b % cp.kv_heads);
+  } else {
+    const int d = b - n_chunk_wg;
+    dec::decode_wg<ACT, KV, HD, pre::kWaves>(dp, sm.d, d % dp.n_rows, d / dp.n_rows, 0);
+  }
+}
+
 }  // namespace
 
+hipError_t attention_ragged_prefill(const DecodeParams& d, const ChunkParams& c, bool wide, int act_dtype,
+                                    int kv_dtype, hipStream_t s) {
+  const int64_t n = static_cast<int64_t>(c.n_items + d.n_rows) * c.kv_heads;
+  if (n <= 0) return hipSuccess;
+  if (n > 0x7fffffff || d.kv_heads != c.kv_heads || d.head_dim != c.head_dim || !d.items ||
+      (wide && c.head_dim != 64))
+    return hipErrorInvalidValue;
+  const dim3 grid(static_cast<unsigned>(n));
+  return with_dtype(act_dtype, [&](auto a) {
+    return with_dtype16(kv_dtype, [&](auto k) {
+      using ACT = decltype(a);
+      using KV = decltype(k);
+      if (c.head_dim == 128) ragged_prefill_kernel<ACT, KV, 128, 1><<<grid, pre::kThreads, 0, s>>>(d, c);
+      else if (wide) ragged_prefill_kernel<ACT, KV, 64, 2><<<grid, pre::kThreads, 0, s>>>(d, c);
+      else ragged_prefill_kernel<ACT, KV, 64, 1><<<grid, pre::kThreads, 0, s>>>(d, c);
+      return hipGetLastError();
+    });
+  });
+}
 
 hipError_t attention_ragged(const DecodeParams& d, const ChunkParams& c, int act_dtype, int kv_dtype,
                             hipStream_t s) {

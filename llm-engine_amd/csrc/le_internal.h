@@ -141,8 +141,20 @@ struct ChunkParams {
 
 hipError_t attention_chunk(const ChunkParams& p, int act_dtype, int kv_dtype, hipStream_t stream);
 
+// Chunk rows as prefill tiles (attention_prefill.hip; 16-bit caches): an item
+// holds prefill_rows() consecutive rows, its block ids are read from the
+// step's tables. A plan whose chunk items are such tiles leaves
+// cfg.chunk_q_tile at kPrefillTiles or kWidePrefillTiles (an explicit row tile
+// is 16 or 32; as an input, both mean the default).
+constexpr int kPrefillTiles = 0, kWidePrefillTiles = -1;
+constexpr int prefill_cols(bool wide) { return wide ? 256 : 128; }  // query columns of a tile
+constexpr int prefill_rows(bool wide, int group) { return prefill_cols(wide) / group; }
+hipError_t attention_prefill(const ChunkParams& p, bool wide, int act_dtype, int kv_dtype, hipStream_t stream);
+
 // A mixed step's chunk rows and decode rows (plan items) in one
 // launch: chunk workgroups first, then decode workgroups.
+hipError_t attention_ragged_prefill(const DecodeParams& d, const ChunkParams& c, bool wide, int act_dtype,
+                                    int kv_dtype, hipStream_t stream);
 hipError_t attention_ragged(const DecodeParams& d, const ChunkParams& c, int act_dtype, int kv_dtype,
                             hipStream_t stream);
 

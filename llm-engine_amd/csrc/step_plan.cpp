@@ -16,7 +16,9 @@
 // slice (a prefill chunk) are cut into tiles of chunk_q_tile consecutive
 // positions; each tile's keys 0..last position are cut into partitions of
 // ~chunk_partition_tokens, one ChunkItem each, run on MFMA tiles (16-bit
-// operands with a bf16/fp16 cache, fp32 operands with an fp32 cache). Split
+// operands with a bf16/fp16 cache, fp32 operands with an fp32 cache). With a
+// 16-bit cache and neither size given, the tiles are prefill tiles instead
+// (cut_prefill below). Split
 // rows of either kind are merged inside their launch by the last partition
 // to finish.
 #include <hip/hip_runtime.h>
@@ -45,6 +47,14 @@ constexpr int kDefaultChunkTile = 32;        // query rows per chunk item (two M
 constexpr int kDefaultChunkPartition = 384;
 constexpr int kMaxChunkParts = 16;           // partitions of a chunk tile the in-kernel merge stages
 constexpr int kMaxChunkItemBlocks = 1024;
+constexpr int64_t kPrefillSlots = 512;       // prefill workgroups in flight: two per CU
+constexpr int64_t kSmallPrefill = 128;       // prefill workgroups of a small step
+constexpr int kSmallPrefillPart = 256;       // its smallest partition
+constexpr int kPrefillSplitKeys = 576;       // shortest prefill tile worth splitting
+constexpr int kMixedPrefillPartition = 1024; // decode rows beside prefill tiles: smallest automatic partition
+constexpr int64_t kSmallPrefillScratch = 8 << 20;  // bytes of partials a small step may use
+constexpr int64_t kFinerPrefillScratch = 24 << 20;  // bytes of the tiles' partials up to which decode rows split finer
+constexpr int64_t kArrivalCounters = 65536;  // (row, kv head) arrival counters of a workspace
 constexpr int kXcds = 8;                     // MI355X: XCDs, each with its own L2
 constexpr int kItemOverheadBlocks = 8;       // a decode item's fixed cost, in streamed blocks    // block ids of one chunk item the kernel stages
 
@@ -124,6 +134,94 @@ std::vector<le::ChunkItem> place_chunk_items(const std::vector<le::ChunkItem>& c
       [](const le::ChunkItem& c) { return static_cast<int64_t>(c.blk_end - c.blk_begin); }, pad);
 }
 
+// ---- prefill tiles (attention_prefill_wg.h) ----
+// How a step's chunk rows are cut for the prefill kernel: tiles of `rows`
+// query rows, partitions of about `part` keys (0: no tile is split).
+struct PrefillCut {
+  bool on = false, wide = false;
+  int rows = 0;
+  int64_t part = 0;
+  int64_t bytes = 0;  // at most this much for the tiles' partials
+  // Partitions (whole blocks) of a tile over nb key blocks of bs: with `part`
+  // at least kDefaultChunkPartition, never more than the 32-row tiles take.
+  int parts(int64_t nb, int bs) const {
+    if (part == 0 || nb * bs <= kPrefillSplitKeys) return 1;
+    const int64_t pb = std::max((part + bs - 1) / bs, (nb + kMaxChunkParts - 1) / kMaxChunkParts);
+    return static_cast<int>((nb + pb - 1) / pb);
+  }
+};
+
+template <typename F>  // f(key blocks of the tile)
+void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
+  for (int i = 0; i < n; i++)
+    if (s[i].len > 1)
+      for (int q0 = 0; q0 < s[i].len; q0 += rows) f((s[i].start + std::min(q0 + rows, s[i].len) + bs - 1) / bs);
+}
+
+// Steps with a 16-bit cache and no explicit tile or partition size: the
+// prefill kernel is the faster one over all of them (32-row tiles against
+// prefill tiles, us: 64 rows after 8000 keys, 32/4 heads x 64, 64 and 29; 4096
+// rows after 0-1536, 131 and 63; 2048 rows after 8192, 32/8 x 128, 845 and 357;
+// 512 rows after 1024, 14/2 x 64, 18.5 and 15.4; even at 1-64 rows after
+// nothing, 10 and 10).
+// * wide tiles (256 columns, head_dim 64): the K/V fragments a wave reads
+//   from LDS serve twice the columns, but a tile takes longer and there are
+//   half as many. Better from about 1000 keys per slot on (8 x 512 rows after
+//   4096, 32/4 heads: 163 against 182 us; 4 x 512 after 1024: 42 against 38).
+// * partitions: none when the tiles alone give three workgroups for every
+//   four slots; otherwise the smallest partition that fits every workgroup
+//   into the slots (the padding of the XCD placement counted), at least 384
+//   keys: a split costs its partials' round trip (8 x 512 rows after 2048
+//   keys: 97 us whole, 138 in 1024-key partitions). Small steps, with at most
+//   kSmallPrefill workgroups, go down to 256 keys (16 rows after 1000 keys:
+//   13.6 against 15.5 us; 2 x 512 rows beside 32 decode rows lose: 44 against
+//   38 for two layers).
+// Steps with more rows than arrival counters keep the 32-row tiles: a step
+// that splits nothing there runs without a workspace.
+PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok) {
+  PrefillCut c;
+  const int group = cfg.q_heads / cfg.kv_heads, bs = cfg.block_size;
+  if (cfg.chunk_q_tile > 0 || cfg.chunk_partition_tokens > 0 || cfg.kv_dtype == LE_F32 ||
+      (cfg.flags & LE_PLAN_TWO_LAUNCHES) || (cfg.head_dim != 64 && cfg.head_dim != 128) || group < 1 || group > 8 ||
+      n_tok * cfg.kv_heads > kArrivalCounters)
+    return c;
+  int64_t tiles = 0, longest = 0;
+  auto total_keys = [&] {  // times kv heads
+    int64_t nb = 0;
+    tiles = 0;
+    for_prefill_tiles(s, n, c.rows, bs, [&](int64_t b) {
+      nb += b;
+      longest = std::max(longest, b);
+      tiles++;
+    });
+    return nb * bs * cfg.kv_heads;
+  };
+  c.rows = le::prefill_rows(true, group);
+  int64_t keys = total_keys();
+  if (tiles == 0) return c;
+  c.on = true;
+  c.wide = cfg.head_dim == 64 && keys >= 1000 * kPrefillSlots;
+  c.rows = le::prefill_rows(c.wide, group);
+  if (!c.wide) keys = total_keys();
+  if (tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
+  const int64_t padded = cfg.kv_heads % kXcds == 0 ? tiles : (tiles + kXcds - 1) / kXcds * kXcds;
+  auto workgroups = [&] {  // with partitions of c.part keys; sets c.bytes
+    int64_t items = 0, rows = 0;
+    for_prefill_tiles(s, n, c.rows, bs, [&](int64_t b) {
+      const int J = c.parts(b, bs);
+      items += J;
+      if (J > 1) rows += c.rows * J;
+    });
+    c.bytes = rows * cfg.q_heads * (cfg.head_dim * 4 + 8);
+    return (items * padded + tiles - 1) / tiles * cfg.kv_heads;
+  };
+  c.part = kSmallPrefillPart;
+  if (workgroups() <= kSmallPrefill && c.bytes <= kSmallPrefillScratch) return c;
+  c.part = std::max<int64_t>((keys / kPrefillSlots + 63) / 64 * 64, kDefaultChunkPartition);
+  while (workgroups() > kPrefillSlots && c.part < longest * bs) c.part += (c.part / 8 + 63) / 64 * 64;
+  return c;
+}
+
 }  // namespace
 
 extern "C" {
@@ -141,47 +239,7 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
   const bool fixed = cfg.table_capacity > 0;
   if (fixed && cfg.partition_tokens <= 0) return LE_EINVAL;
   const int bs = cfg.block_size;
-  if (!fixed && cfg.partition_tokens <= 0) {
-    // Size decode partitions so the step has about kTargetItems workgroups,
-    // two per CU. Each workgroup pays a fixed chain of dependent memory
-    // round trips (block ids, then K/V; partial store, arrival counter, merge)
-    // of several microseconds, so on MI355X a few long partitions stream
-    // faster than many short ones (measured: 64 x 4096 rows, 2048-token
-    // partitions 4.1 TB/s, 256-token 2.2 TB/s; config 2, 640-768 tokens
-    // 16.3 us, 1024 17.1 us, 512 18.0 us).
-    int64_t ctx = 0;
-    for (int i = 0; i < n_slices; i++)
-      if (slices[i].len == 1)
-        for (int r = 0; r < slices[i].len; r++) ctx += slices[i].start + r + 1;
-    const int64_t per_kvh = std::max<int64_t>(1, kTargetItems / cfg.kv_heads);
-    int64_t part = (ctx + per_kvh - 1) / per_kvh;
-    part = (part + kPartitionQuantum - 1) / kPartitionQuantum * kPartitionQuantum;
-    part = std::max<int64_t>(part, kDefaultPartition);
-    // In a mixed step the chunk workgroups hold most CUs for the first half
-    // of the launch; splitting the decode rows further only adds merges
-    // (config 3: 22.7 us with the rule above, 22.4 us with 2048 tokens).
-    bool chunk_rows = false;
-    for (int i = 0; i < n_slices; i++) chunk_rows |= slices[i].len > 1;
-    if (chunk_rows) {
-      part = std::max<int64_t>(part, kMixedStepPartition);
-    } else {
-      // The rows' partitions are whole ceilings, so the rule above can
-      // overshoot: grow the partition until the step's workgroups fit one
-      // round at two per CU (TinyLlama-shaped decode steps, 64 rows, 4 kv
-      // heads: 136-144 items per kv head ran 20.6-21.5 us per launch, 120
-      // items 15-16 us).
-      const int max_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
-      auto items_at = [&](int64_t pt) {
-        const int64_t pb = (pt + bs - 1) / bs;
-        int64_t n = 0;
-        for (int i = 0; i < n_slices; i++)
-          if (slices[i].len == 1) n += std::min<int64_t>((slices[i].start / bs + 1 + pb - 1) / pb, max_parts);
-        return n;
-      };
-      while (part < kMaxAutoPartition && items_at(part) * cfg.kv_heads > kTargetItems) part += kPartitionQuantum;
-    }
-    cfg.partition_tokens = static_cast<int32_t>(std::min<int64_t>(part, kMaxAutoPartition));
-  }
+  const le_plan_config asked = cfg;
   if (cfg.chunk_q_tile <= 0) cfg.chunk_q_tile = kDefaultChunkTile;
   // 384 keys: one LDS stage of a 16-bit cache, three of fp32 at head_dim 64
   // (config 3 with fp32 K/V, 24 layers: 1.18 ms per step, against 1.62 with
@@ -189,11 +247,6 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
   if (cfg.chunk_partition_tokens <= 0)
     cfg.chunk_partition_tokens = kDefaultChunkPartition;
   if (cfg.chunk_q_tile != 16 && cfg.chunk_q_tile != 32) return LE_EUNSUPPORTED;  // MFMA row tiles
-  const int dec_pb = round_to_blocks(cfg.partition_tokens, bs);
-  const int chk_pb = round_to_blocks(cfg.chunk_partition_tokens, bs);
-  const bool mfma_chunks = true;  // chunk rows on MFMA tiles, every cache type
-  const int max_decode_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
-
   // ---- sizes, and validation of every slice against its table ----
   int64_t n_tok = 0, n_table = 0;
   int n_logits = 0, n_seqs = 0, max_pos = 0;
@@ -229,6 +282,59 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     max_pos = std::max(max_pos, last);
   }
   if (n_tok > INT32_MAX / 2) return LE_EUNSUPPORTED;
+  const PrefillCut pre = cut_prefill(asked, slices, n_slices, n_tok);
+  if (!fixed && cfg.partition_tokens <= 0) {
+    // Size decode partitions so the step has about kTargetItems workgroups,
+    // two per CU. Each workgroup pays a fixed chain of dependent memory
+    // round trips (block ids, then K/V; partial store, arrival counter, merge)
+    // of several microseconds, so on MI355X a few long partitions stream
+    // faster than many short ones (measured: 64 x 4096 rows, 2048-token
+    // partitions 4.1 TB/s, 256-token 2.2 TB/s; config 2, 640-768 tokens
+    // 16.3 us, 1024 17.1 us, 512 18.0 us).
+    int64_t ctx = 0;
+    for (int i = 0; i < n_slices; i++)
+      if (slices[i].len == 1)
+        for (int r = 0; r < slices[i].len; r++) ctx += slices[i].start + r + 1;
+    const int64_t per_kvh = std::max<int64_t>(1, kTargetItems / cfg.kv_heads);
+    int64_t part = (ctx + per_kvh - 1) / per_kvh;
+    part = (part + kPartitionQuantum - 1) / kPartitionQuantum * kPartitionQuantum;
+    part = std::max<int64_t>(part, kDefaultPartition);
+    // In a mixed step the chunk workgroups hold most CUs for the first half
+    // of the launch; splitting the decode rows further only adds merges
+    // (config 3: 22.7 us with the rule above, 22.4 us with 2048 tokens).
+    bool chunk_rows = false;
+    for (int i = 0; i < n_slices; i++) chunk_rows |= slices[i].len > 1;
+    if (chunk_rows) {
+      // (beside prefill tiles, whose workgroups share a CU with the decode
+      // rows', 1024: 2 x 512 rows after 1024 keys and 32 decode rows 25.6
+      // against 31.1 us). Those partitions need at most 5 MB more of partials
+      // than 2048-key ones: where the tiles' own leave that much of the static
+      // scratch, else 2048 as before.
+      const bool finer = pre.on && pre.bytes <= kFinerPrefillScratch;
+      part = std::max<int64_t>(part, finer ? kMixedPrefillPartition : kMixedStepPartition);
+    } else {
+      // The rows' partitions are whole ceilings, so the rule above can
+      // overshoot: grow the partition until the step's workgroups fit one
+      // round at two per CU (TinyLlama-shaped decode steps, 64 rows, 4 kv
+      // heads: 136-144 items per kv head ran 20.6-21.5 us per launch, 120
+      // items 15-16 us).
+      const int max_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
+      auto items_at = [&](int64_t pt) {
+        const int64_t pb = (pt + bs - 1) / bs;
+        int64_t n = 0;
+        for (int i = 0; i < n_slices; i++)
+          if (slices[i].len == 1) n += std::min<int64_t>((slices[i].start / bs + 1 + pb - 1) / pb, max_parts);
+        return n;
+      };
+      while (part < kMaxAutoPartition && items_at(part) * cfg.kv_heads > kTargetItems) part += kPartitionQuantum;
+    }
+    cfg.partition_tokens = static_cast<int32_t>(std::min<int64_t>(part, kMaxAutoPartition));
+  }
+  const int dec_pb = round_to_blocks(cfg.partition_tokens, bs);
+  const int chk_pb = round_to_blocks(cfg.chunk_partition_tokens, bs);
+  const bool mfma_chunks = true;  // chunk rows on MFMA tiles, every cache type
+  const int max_decode_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
+
   // Fixed layout: every row owns parts_cap partial slots and every table
   // table_capacity entries, whatever its current length.
   const int parts_cap = fixed ? std::min((cfg.table_capacity + dec_pb - 1) / dec_pb, max_decode_parts) : 0;
@@ -253,14 +359,15 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     for (int i = 0; i < n_slices; i++) {
       const le_step_slice& s = slices[i];
       if (s.len > 1 && mfma_chunks) {
-        for (int q0 = 0; q0 < s.len; q0 += cfg.chunk_q_tile) {
-          const int nq = std::min(cfg.chunk_q_tile, s.len - q0);
+        const int rows = pre.on ? pre.rows : cfg.chunk_q_tile;
+        for (int q0 = 0; q0 < s.len; q0 += rows) {
+          const int nq = std::min(rows, s.len - q0);
           const int last = s.start + q0 + nq - 1;
           const int nb = last / bs + 1;
           // Long contexts get longer partitions rather than more of them.
           const int pb = std::max(chk_pb, (nb + kMaxChunkParts - 1) / kMaxChunkParts);
           if (pb > kMaxChunkItemBlocks) return LE_EUNSUPPORTED;  // the kernel stages an item's ids in LDS
-          const int J = (nb + pb - 1) / pb;
+          const int J = pre.on ? pre.parts(nb, bs) : (nb + pb - 1) / pb;
           const int base = J > 1 ? parts : -1;
           for (int j = 0; j < J; j++) {
             le::ChunkItem c{};
@@ -323,7 +430,9 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
   }
   bool chunk_split = false;
   for (const auto& c : chk) chunk_split |= c.part0 >= 0;
-  if (chunk_split) {
+  // Prefill workgroups are numbered with the kv heads innermost: with a
+  // multiple of 8 of them, one head's tiles share an XCD in any order.
+  if (chunk_split && !(pre.on && cfg.kv_heads % kXcds == 0)) {
     chk = place_chunk_items(chk);
   } else {
     std::stable_sort(chk.begin(), chk.end(), [](const le::ChunkItem& a, const le::ChunkItem& b) {
@@ -346,6 +455,10 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
   // ---- layout: every array 256-byte aligned in one buffer ----
   le_step_plan P{};
   P.cfg = cfg;
+  if (pre.on) {
+    P.cfg.chunk_q_tile = pre.wide ? le::kWidePrefillTiles : le::kPrefillTiles;
+    P.cfg.chunk_partition_tokens = 0;
+  }
   P.n_tokens = static_cast<int32_t>(n_tok);
   P.n_seqs = n_seqs;
   P.n_table = static_cast<int32_t>(n_table);

@@ -1,0 +1,94 @@
+"""GPU parity of the prefill tiles (attention_prefill_wg.h) with the oracle at
+the edges of their tiles, partitions and softmax base."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from cases import make_case
+from gpu_util import emulated_bar, max_abs, oracle_out, poison_unused
+from llm_engine_amd._lib import LE_PLAN_XCD_LOCAL
+from test_gpu_attention import run_ragged, within
+
+pytestmark = pytest.mark.gpu
+
+# 16-bit activations round the output once more (2^-9 and 2^-12 relative,
+# doubled for the error carried into it)
+OUT_REL = {"f32": 0.0, "bf16": 2.0 ** -8, "f16": 2.0 ** -11}
+ACT = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}
+
+
+def check(case, act, gpu, want_split=None, want_wide=False, bar=None, flags=LE_PLAN_XCD_LOCAL):
+    got, qh, plan = run_ragged(case, ACT[act], gpu, flags=flags)
+    assert plan.plan.cfg.chunk_q_tile == (-1 if want_wide else 0)
+    if want_split is not None:
+        assert (plan.plan.n_parts > 0) == want_split
+    want = oracle_out(case, qh)
+    tol = emulated_bar(case, qh, want) if bar is None else bar(qh, want)
+    err = np.abs(got.astype(np.float64) - want)
+    print(f"prefill {case.q_heads}/{case.kv_heads}x{case.head_dim} bs {case.block_size} rows {case.n_tokens} "
+          f"items {plan.plan.n_chunk_items} parts {plan.plan.n_parts}: max|err| {err.max():.3e} tol {tol:.3e}")
+    assert np.isfinite(got).all() and (err <= tol + OUT_REL[act] * np.abs(want)).all()
+    return got
+
+
+# rows of a 128-column tile: 18 (G 7), 16 (G 8), 128 (G 1), 32 (G 4); keys at
+# the edges of the 64-key tiles, of a block and of the causal diagonal
+@pytest.mark.parametrize("heads,kv,act,bs", [((14, 2, 64), "bf16", "bf16", 16), ((32, 4, 64), "f16", "f16", 8),
+                                             ((3, 3, 64), "bf16", "f32", 32), ((32, 8, 128), "bf16", "bf16", 16),
+                                             ((7, 1, 128), "f16", "f32", 64), ((10, 2, 64), "bf16", "f32", 16)])
+def test_prefill_tile_edges(gpu, heads, kv, act, bs):
+    H, KH, hd = heads
+    tile = 128 // (H // KH)
+    q_len = [2, tile - 1, tile, tile + 1, 65, 7, 3, 1, 1]
+    ctx = [2, tile - 1, tile + 62, tile + 64, 130, 64, 68, 40, 333]
+    ctx = [max(a, b) for a, b in zip(ctx, q_len)]
+    case = make_case(ctx, H, KH, hd, bs, q_len=q_len, seed=H, kv_bf16=kv == "bf16", kv_f16=kv == "f16")
+    poison_unused(case)
+    check(case, act, gpu, want_split=False)
+
+
+# tiles split over partitions (their merge, of 2 to 16 partials), with XCD-local
+# and with write-through partials, beside split decode rows
+@pytest.mark.parametrize("flags", [0, LE_PLAN_XCD_LOCAL])
+@pytest.mark.parametrize("heads,kv", [((14, 2, 64), "bf16"), ((8, 8, 128), "bf16"), ((32, 4, 64), "f16")])
+def test_prefill_split_tiles(gpu, heads, kv, flags):
+    H, KH, hd = heads
+    case = make_case([577, 1500, 700, 6000, 1100, 2500], H, KH, hd, 16, q_len=[5, 40, 33, 3, 1, 1], seed=3,
+                     kv_bf16=kv == "bf16", kv_f16=kv == "f16")
+    check(case, "f32", gpu, want_split=True, flags=flags)
+
+
+def test_prefill_wide_tiles(gpu):
+    """256-column tiles: a step past 1000 keys per workgroup slot. The bar is
+    twice the error of the 32-row tiles, which make the same roundings."""
+    case = make_case([16100, 15000], 32, 4, 64, 16, q_len=[300, 45], seed=4, kv_bf16=True)
+
+    def bar(qh, want):
+        old, _, plan = run_ragged(case, torch.float32, gpu, chunk_q_tile=32)
+        assert plan.plan.cfg.chunk_q_tile == 32
+        return 2 * max_abs(old, want)
+
+    check(case, "f32", gpu, want_wide=True, want_split=True, bar=bar)
+
+
+@pytest.mark.parametrize("kind", ["large", "negative", "rising"])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_prefill_softmax_base(gpu, kind, hd):
+    """Scores far from 0 (the base that they are taken relative to starts at
+    0): tens of log2 units wide, all far below 0, and rising along the keys so
+    that the base moves tile after tile."""
+    case = make_case([300, 150], 8, 2, hd, 16, q_len=[200, 33], seed=5)
+    pos = np.zeros(case.k_cache.shape[0])
+    for s in range(2):
+        p = np.arange([300, 150][s])
+        pos[case.blocks_of(s)[p // 16].astype(np.int64) * 16 + p % 16] = p
+    k = case.k_cache.reshape(-1, 2, hd)
+    q = case.q.reshape(-1, 8, hd)
+    if kind == "large":
+        k *= 8.0
+    else:
+        q[..., 0] = 8.0
+        k[..., 0] = (-12.0 if kind == "negative" else pos[:, None] / 16)
+    case.k_cache, case.v_cache = (oracle.f32_to_bf16(c) for c in (case.k_cache, case.v_cache))
+    check(case, "f32", gpu)

@@ -1,0 +1,113 @@
+"""How a step's chunk rows are cut into prefill tiles (16-bit caches, neither
+tile nor partition given): the work lists against the step, and against the
+32-row tiles of the same step (chunk_q_tile given), over head groups, block
+sizes, ragged rows, repeated sequences and step sizes."""
+import numpy as np
+import pytest
+import torch
+
+from llm_engine_amd import kernels
+from llm_engine_amd._lib import LE_PLAN_TWO_LAUNCHES, LE_PLAN_XCD_LOCAL
+
+
+def items_of(plan):
+    P = plan.plan
+    return plan.host.numpy()[P.off_chunk_items:P.off_chunk_items + 36 * P.n_chunk_items].view(np.int32).reshape(-1, 9)
+
+
+def step(rng, bs, n_chunks, max_rows, max_hist, n_decode):
+    out = []
+    for i in range(n_chunks + n_decode):
+        ln = int(rng.integers(2, max_rows + 1)) if i < n_chunks else 1
+        start = int(rng.integers(0, max_hist + 1))
+        nb = (start + ln + bs - 1) // bs
+        out.append(kernels.Slice(i, start, ln, True, rng.permutation(nb + 3).astype(np.int32)[:nb],
+                                 np.zeros(start + ln, np.int32)))
+    return out
+
+
+SHAPES = [(14, 2, 64), (32, 4, 64), (16, 16, 64), (32, 8, 128), (28, 4, 128), (6, 2, 64), (8, 1, 128)]
+
+
+@pytest.mark.parametrize("heads", SHAPES)
+@pytest.mark.parametrize("bs", [8, 16, 64, 512])
+def test_prefill_tiles_cover_the_step(heads, bs):
+    H, KH, hd = heads
+    rng = np.random.default_rng(H * 1000 + bs)
+    wide = 0
+    for n_chunks, max_rows, max_hist, n_decode in [(1, 2, 0, 0), (1, 40, 100, 3), (3, 300, 1500, 0), (2, 17, 9000, 5),
+                                                   (8, 512, 1536, 0), (4, 600, 20000, 9), (1, 3, 16000, 0)]:
+        sl = step(rng, bs, n_chunks, max_rows, max_hist, n_decode)
+
+        def make(**kw):
+            return kernels.Plan(sl, H, KH, hd, bs, torch.bfloat16, device="cpu", pin=False, **kw)
+
+        plan, tiles32 = make(flags=LE_PLAN_XCD_LOCAL), make(flags=LE_PLAN_XCD_LOCAL, chunk_q_tile=32)
+        P, old = plan.plan, tiles32.plan
+        assert P.cfg.chunk_q_tile <= 0 and old.cfg.chunk_q_tile == 32
+        is_wide = P.cfg.chunk_q_tile < 0
+        wide += is_wide
+        cols = 256 if is_wide else 128
+        assert hd == 64 or not is_wide
+        pos, tables = plan.host_array("positions"), plan.host_array("tables")
+        toff, items = plan.host_array("table_offset"), items_of(plan)
+        stride = P.decode_ids_stride
+        n_ids = P.n_decode_items + P.n_chunk_items
+        ids = plan.host.numpy()[P.off_decode_ids:P.off_decode_ids + 4 * n_ids * stride].view(np.int32).reshape(-1, stride)
+        by_tile, owned, bins = {}, [], {}
+        for k, it in enumerate(items):
+            tb, nq, b0, b1, p0, J, seq, part, live = (int(x) for x in it)
+            if nq == 0:
+                continue
+            assert 1 <= nq * (H // KH) <= cols and (np.diff(pos[tb:tb + nq]) == 1).all()
+            assert b1 > b0 and live == min((b1 - b0) * bs, pos[tb + nq - 1] + 1 - b0 * bs) and live >= 1
+            row = ids[P.n_decode_items + k]
+            assert (row[:b1 - b0] == tables[toff[seq] + b0:toff[seq] + b1]).all() and (row[b1 - b0:] == -1).all()
+            by_tile.setdefault(tb, []).append((b0, b1, p0, J, part, nq))
+            if J > 1:
+                owned += [p0 + r * J for r in range(nq)]
+                bins.setdefault(tb, set()).add(k % 8 if KH % 8 else 0)
+            else:
+                assert p0 == -1
+        assert all(len(b) == 1 for b in bins.values())  # one tile's partitions on one XCD
+        rows = set()
+        for tb, parts in by_tile.items():
+            parts.sort()
+            nq = parts[0][5]
+            assert parts[0][0] == 0 and parts[-1][1] == pos[tb + nq - 1] // bs + 1
+            assert all(a[1] == b[0] for a, b in zip(parts, parts[1:])) and len(parts) == parts[0][3] <= 16
+            assert [p[4] for p in parts] == list(range(len(parts)))
+            rows |= set(range(tb, tb + nq))
+        chunk_rows = sum(s.len for s in sl if s.len > 1)
+        assert rows == set(range(chunk_rows))  # chunks first in these steps
+        dec = plan.host.numpy()[P.off_decode_items:P.off_decode_items + 32 * P.n_decode_items].view(np.int32).reshape(-1, 8)
+        owned += [int(d[5]) for d in dec if d[5] >= 0]
+        assert sorted(owned) == list(range(P.n_parts))
+        # scratch: no more than the 32-row tiles take, or a small step's bound
+        # (8 MiB for the tiles and 5 MB for finer decode partitions)
+        row_bytes = H * (hd * 4 + 8)
+        assert P.n_parts * row_bytes <= max(old.n_parts * row_bytes + 5_000_000, (8 << 20) + 5_000_000)
+        assert P.n_parts * row_bytes <= max(old.n_parts * row_bytes, 31 << 20)
+    assert wide > 0 or heads != (32, 4, 64)  # both widths were seen
+
+
+def test_prefill_tiles_only_where_asked_for_nothing():
+    """Explicit sizes, the two-launch flag, fp32 caches and steps without
+    arrival counters for every row keep the 32-row tiles; a plan's own
+    resolved configuration gives the same plan again."""
+    sl = step(np.random.default_rng(1), 16, 2, 400, 900, 3)
+
+    def make(kv=torch.bfloat16, heads=(14, 2, 64), slices=sl, **kw):
+        return kernels.Plan(slices, *heads, 16, kv, device="cpu", pin=False, **kw).plan
+
+    auto = make()
+    assert auto.cfg.chunk_q_tile <= 0 and auto.cfg.chunk_partition_tokens == 0
+    again = make(chunk_q_tile=auto.cfg.chunk_q_tile, chunk_partition_tokens=auto.cfg.chunk_partition_tokens,
+                 partition_tokens=auto.cfg.partition_tokens)
+    assert (again.n_chunk_items, again.n_parts, again.bytes) == (auto.n_chunk_items, auto.n_parts, auto.bytes)
+    for kw in (dict(chunk_q_tile=32), dict(chunk_q_tile=16), dict(chunk_partition_tokens=256),
+               dict(flags=LE_PLAN_TWO_LAUNCHES), dict(kv=torch.float32)):
+        assert make(**kw).cfg.chunk_q_tile in (16, 32)
+    many = [kernels.Slice(i, 0, 600, True, np.arange(38, dtype=np.int32), np.zeros(600, np.int32)) for i in range(7)]
+    assert make(heads=(16, 16, 64), slices=many).cfg.chunk_q_tile == 32  # 4200 rows x 16 kv heads
+    assert make(heads=(16, 16, 64), slices=many[:6]).cfg.chunk_q_tile <= 0
