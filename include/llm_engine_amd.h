@@ -151,7 +151,7 @@ typedef struct le_plan_config {
   int32_t kv_dtype;            /* le_dtype of the cache the plan will be run against */
   int32_t partition_tokens;    /* split-K partition of decode rows; 0 = default */
   int32_t chunk_q_tile;        /* query rows per chunk tile (16 or 32); 0 (or less) = default: 32
-                                  with an fp32 cache, else tiles of 128 or 256 query columns
+                                  with an fp32 cache of head_dim 128, else tiles of 128 or 256 query columns
                                   (row, head), sized and partitioned by the step; a packed plan's
                                   cfg then holds 0 or -1 here and 0 below */
   int32_t chunk_partition_tokens; /* key partition of chunk tiles; 0 = default */

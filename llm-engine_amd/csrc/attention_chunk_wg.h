@@ -11,7 +11,8 @@
 // row; here 32 consecutive rows share every K/V read. With a 16-bit cache
 // these tiles run where a plan names their row tile or partition, asks for two
 // launches, or has more rows than arrival counters; the prefill tiles
-// (attention_prefill_wg.h) run everywhere else.
+// (attention_prefill_wg.h) run everywhere else. With an fp32 cache of head_dim 64 the same holds
+// (attention_prefill_f32_wg.h); with one of head_dim 128 they always run.
 //
 // gfx950 design:
 //   * one 512-thread workgroup (8 waves) per (32-row tile, kv head, key

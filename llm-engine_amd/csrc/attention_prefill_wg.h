@@ -107,6 +107,96 @@ __device__ __forceinline__ void gather8(const f32x16& acc, int e, float scale, f
   }
 }
 
+// The end of a tile: its output, or its partial and, in the last partition to
+// arrive, the merge. Column tile nc of a lane holds query row row_of[nc] (-1:
+// none) and head head_of[nc], accumulators acc less base, and the lane's half
+// of the row sum.
+template <typename ACT, typename KV, int HD, int NC>
+__device__ __forceinline__ void finish_tile(const ChunkParams& p, const ChunkItem& it, int kvh, int& last,
+                                            f32x16 (&acc)[NC][HD / 32], float (&base)[NC], float (&lsum)[NC],
+                                            int (&row_of)[NC], int (&head_of)[NC]) {
+  constexpr int DT = HD / 32;
+  const int tid = threadIdx.x, half = (tid & (kWave - 1)) >> 5;
+  const int G = p.q_heads / p.kv_heads;
+  // acc[nc][d][e] = O[column][dim 32 d + 8 (e / 4) + 4 half + e % 4]
+  float l_tot[NC];
+#pragma unroll
+  for (int nc = 0; nc < NC; nc++) l_tot[nc] = halves_sum(lsum[nc]);
+  if (it.part0 < 0) {
+#pragma unroll
+    for (int nc = 0; nc < NC; nc++) {
+      ACT* out = static_cast<ACT*>(p.out) +
+                 (static_cast<int64_t>(it.tok_begin + max(row_of[nc], 0)) * p.q_heads + head_of[nc]) * HD + half * 8;
+      const float inv = 1.f / l_tot[nc];
+#pragma unroll
+      for (int d = 0; d < DT; d++)
+#pragma unroll
+        for (int e = 0; e < 16; e += 8) {
+          float f[8];
+          gather8(acc[nc][d], e, inv, f);  // every lane takes part in the exchange
+          if (row_of[nc] >= 0) elem<ACT>::store8(out + d * 32 + e * 2, f);
+        }
+    }
+    return;
+  }
+
+  // ---- split tile: the partial in the chunk kernel's record layout, then
+  // the last partition to arrive merges ----
+  const int64_t rec_tile = static_cast<int64_t>(it.part0 - it.part) * p.q_heads;
+  const __amdgpu_buffer_rsrc_t acc_rsrc = coherent_rsrc(p.parts.acc + rec_tile * HD);
+  float* ml = reinterpret_cast<float*>(p.parts.ml);
+#pragma unroll
+  for (int nc = 0; nc < NC; nc++) {
+    const bool on = row_of[nc] >= 0;
+    const int64_t rec = static_cast<int64_t>(it.part0 + max(row_of[nc], 0) * it.part_stride) * p.q_heads + head_of[nc];
+    const float inv = l_tot[nc] > 0.f ? 1.f / l_tot[nc] : 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; d++)
+#pragma unroll
+      for (int e = 0; e < 16; e += 8) {
+        float f[8];
+        gather8(acc[nc][d], e, inv, f);
+        if (!on) continue;
+        const int64_t el = (rec - rec_tile) * HD + d * 32 + e * 2 + half * 8;
+        if constexpr (chk::kHalfPartials<KV>) {
+          const uint4 h = make_uint4(pack_f16x2(f[0], f[1]), pack_f16x2(f[2], f[3]), pack_f16x2(f[4], f[5]),
+                                     pack_f16x2(f[6], f[7]));
+          const f32x4v v = __builtin_bit_cast(f32x4v, h);
+          if (p.l2_local) st_l2_16(acc_rsrc, static_cast<uint32_t>(el * 2), v);
+          else st_coherent16(acc_rsrc, static_cast<uint32_t>(el * 2), v);
+        } else {
+#pragma unroll
+          for (int q = 0; q < 2; q++) {
+            const f32x4v v = {f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]};
+            if (p.l2_local) st_l2_16(acc_rsrc, static_cast<uint32_t>((el + 4 * q) * 4), v);
+            else st_coherent16(acc_rsrc, static_cast<uint32_t>((el + 4 * q) * 4), v);
+          }
+        }
+      }
+    if (on && half == 0) {
+      const float m = l_tot[nc] > 0.f ? base[nc] : -FLT_MAX;
+      if (p.l2_local) {
+        reinterpret_cast<float2*>(ml)[rec] = make_float2(m, l_tot[nc]);
+      } else {
+        chk::st_dev(ml + rec * 2, m);
+        chk::st_dev(ml + rec * 2 + 1, l_tot[nc]);
+      }
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores are performed
+  __syncthreads();                // ... and every other thread's
+  arrival_t* counter = p.parts.counters + static_cast<int64_t>(it.tok_begin) * p.kv_heads + kvh;
+  if (tid == 0) {
+    const arrival_t seen = __hip_atomic_fetch_add(counter, arrival_t{1}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    last = seen == static_cast<arrival_t>(it.part_stride - 1);
+  }
+  __syncthreads();
+  if (!last) return;
+  chk::merge_tile<ACT, HD, 4, chk::kHalfPartials<KV>, kThreads, HD == 64 && NC == 1 ? 2 : 4>(p, it, acc_rsrc, ml, rec_tile, it.part0 - it.part,
+                                                               it.part_stride, G, kvh, it.n_q, it.tok_begin);
+  if (tid == 0) __hip_atomic_store(counter, arrival_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // One prefill workgroup: item `item`, kv head `kvh`, NC column tiles a wave.
 template <typename ACT, typename KV, int HD, int NC>
 __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>& sm, int item, int kvh) {
@@ -369,83 +459,7 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
     for (int t = 0; t < n_tiles; t++) step(t, sa, sa);
   }
 
-  // acc[nc][d][e] = O[column][dim 32 d + 8 (e / 4) + 4 half + e % 4]
-  float l_tot[NC];
-#pragma unroll
-  for (int nc = 0; nc < NC; nc++) l_tot[nc] = halves_sum(lsum[nc]);
-  if (it.part0 < 0) {
-#pragma unroll
-    for (int nc = 0; nc < NC; nc++) {
-      ACT* out = static_cast<ACT*>(p.out) +
-                 (static_cast<int64_t>(it.tok_begin + max(row_of[nc], 0)) * p.q_heads + head_of[nc]) * HD + half * 8;
-      const float inv = 1.f / l_tot[nc];
-#pragma unroll
-      for (int d = 0; d < DT; d++)
-#pragma unroll
-        for (int e = 0; e < 16; e += 8) {
-          float f[8];
-          gather8(acc[nc][d], e, inv, f);  // every lane takes part in the exchange
-          if (row_of[nc] >= 0) elem<ACT>::store8(out + d * 32 + e * 2, f);
-        }
-    }
-    return;
-  }
-
-  // ---- split tile: the partial in the chunk kernel's record layout, then
-  // the last partition to arrive merges ----
-  const int64_t rec_tile = static_cast<int64_t>(it.part0 - it.part) * p.q_heads;
-  const __amdgpu_buffer_rsrc_t acc_rsrc = coherent_rsrc(p.parts.acc + rec_tile * HD);
-  float* ml = reinterpret_cast<float*>(p.parts.ml);
-#pragma unroll
-  for (int nc = 0; nc < NC; nc++) {
-    const bool on = row_of[nc] >= 0;
-    const int64_t rec = static_cast<int64_t>(it.part0 + max(row_of[nc], 0) * it.part_stride) * p.q_heads + head_of[nc];
-    const float inv = l_tot[nc] > 0.f ? 1.f / l_tot[nc] : 0.f;
-#pragma unroll
-    for (int d = 0; d < DT; d++)
-#pragma unroll
-      for (int e = 0; e < 16; e += 8) {
-        float f[8];
-        gather8(acc[nc][d], e, inv, f);
-        if (!on) continue;
-        const int64_t el = (rec - rec_tile) * HD + d * 32 + e * 2 + half * 8;
-        if constexpr (chk::kHalfPartials<KV>) {
-          const uint4 h = make_uint4(pack_f16x2(f[0], f[1]), pack_f16x2(f[2], f[3]), pack_f16x2(f[4], f[5]),
-                                     pack_f16x2(f[6], f[7]));
-          const f32x4v v = __builtin_bit_cast(f32x4v, h);
-          if (p.l2_local) st_l2_16(acc_rsrc, static_cast<uint32_t>(el * 2), v);
-          else st_coherent16(acc_rsrc, static_cast<uint32_t>(el * 2), v);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 2; q++) {
-            const f32x4v v = {f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]};
-            if (p.l2_local) st_l2_16(acc_rsrc, static_cast<uint32_t>((el + 4 * q) * 4), v);
-            else st_coherent16(acc_rsrc, static_cast<uint32_t>((el + 4 * q) * 4), v);
-          }
-        }
-      }
-    if (on && half == 0) {
-      const float m = l_tot[nc] > 0.f ? base[nc] : -FLT_MAX;
-      if (p.l2_local) {
-        reinterpret_cast<float2*>(ml)[rec] = make_float2(m, l_tot[nc]);
-      } else {
-        chk::st_dev(ml + rec * 2, m);
-        chk::st_dev(ml + rec * 2 + 1, l_tot[nc]);
-      }
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores are performed
-  __syncthreads();                // ... and every other thread's
-  arrival_t* counter = p.parts.counters + static_cast<int64_t>(it.tok_begin) * p.kv_heads + kvh;
-  if (tid == 0) {
-    const arrival_t seen = __hip_atomic_fetch_add(counter, arrival_t{1}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    last = seen == static_cast<arrival_t>(it.part_stride - 1);
-  }
-  __syncthreads();
-  if (!last) return;
-  chk::merge_tile<ACT, HD, 4, chk::kHalfPartials<KV>, kThreads, HD == 64 && NC == 1 ? 2 : 4>(p, it, acc_rsrc, ml, rec_tile, it.part0 - it.part,
-                                                               it.part_stride, G, kvh, it.n_q, it.tok_begin);
-  if (tid == 0) __hip_atomic_store(counter, arrival_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  finish_tile<ACT, KV, HD, NC>(p, it, kvh, last, acc, base, lsum, row_of, head_of);
 }
 
 }  // namespace

@@ -141,7 +141,7 @@ struct ChunkParams {
 
 hipError_t attention_chunk(const ChunkParams& p, int act_dtype, int kv_dtype, hipStream_t stream);
 
-// Chunk rows as prefill tiles (attention_prefill.hip; 16-bit caches): an item
+// Chunk rows as prefill tiles (attention_prefill.hip; 16-bit caches and fp32 ones of head_dim 64): an item
 // holds prefill_rows() consecutive rows, its block ids are read from the
 // step's tables. A plan whose chunk items are such tiles leaves
 // cfg.chunk_q_tile at kPrefillTiles or kWidePrefillTiles (an explicit row tile

@@ -53,6 +53,8 @@ constexpr int kSmallPrefillPart = 256;       // its smallest partition
 constexpr int kPrefillSplitKeys = 576;       // shortest prefill tile worth splitting
 constexpr int kMixedPrefillPartition = 1024; // decode rows beside prefill tiles: smallest automatic partition
 constexpr int64_t kSmallPrefillScratch = 8 << 20;  // bytes of partials a small step may use
+constexpr int kF32PrefillPart = 128;         // smallest partition of an fp32 prefill tile: two key tiles
+constexpr int64_t kF32PrefillScratch = 16 << 20;    // the same with an fp32 cache
 constexpr int64_t kFinerPrefillScratch = 24 << 20;  // bytes of the tiles' partials up to which decode rows split finer
 constexpr int64_t kArrivalCounters = 65536;  // (row, kv head) arrival counters of a workspace
 constexpr int kXcds = 8;                     // MI355X: XCDs, each with its own L2
@@ -141,11 +143,12 @@ struct PrefillCut {
   bool on = false, wide = false;
   int rows = 0;
   int64_t part = 0;
+  int64_t split_keys = kPrefillSplitKeys;
   int64_t bytes = 0;  // at most this much for the tiles' partials
   // Partitions (whole blocks) of a tile over nb key blocks of bs: with `part`
   // at least kDefaultChunkPartition, never more than the 32-row tiles take.
   int parts(int64_t nb, int bs) const {
-    if (part == 0 || nb * bs <= kPrefillSplitKeys) return 1;
+    if (part == 0 || nb * bs <= split_keys) return 1;
     const int64_t pb = std::max((part + bs - 1) / bs, (nb + kMaxChunkParts - 1) / kMaxChunkParts);
     return static_cast<int>((nb + pb - 1) / pb);
   }
@@ -158,9 +161,9 @@ void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
       for (int q0 = 0; q0 < s[i].len; q0 += rows) f((s[i].start + std::min(q0 + rows, s[i].len) + bs - 1) / bs);
 }
 
-// Steps with a 16-bit cache and no explicit tile or partition size: the
-// prefill kernel is the faster one over all of them (32-row tiles against
-// prefill tiles, us: 64 rows after 8000 keys, 32/4 heads x 64, 64 and 29; 4096
+// Steps with no explicit tile or partition size, with a 16-bit cache or an fp32
+// cache of head_dim 64: the prefill kernel is the faster one over all of them
+// (32-row tiles against prefill tiles, us: 64 rows after 8000 keys, 32/4 heads x 64, 64 and 29; 4096
 // rows after 0-1536, 131 and 63; 2048 rows after 8192, 32/8 x 128, 845 and 357;
 // 512 rows after 1024, 14/2 x 64, 18.5 and 15.4; even at 1-64 rows after
 // nothing, 10 and 10).
@@ -175,13 +178,23 @@ void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
 //   keys: 97 us whole, 138 in 1024-key partitions). Small steps, with at most
 //   kSmallPrefill workgroups, go down to 256 keys (16 rows after 1000 keys:
 //   13.6 against 15.5 us; 2 x 512 rows beside 32 decode rows lose: 44 against
-//   38 for two layers).
+//   38 for two layers). Partitions below 384 keys only while their partials and
+//   the decode rows' stay within kFinerPrefillScratch, so that a step which the
+//   32-row tiles run in the static scratch still does.
+// * an fp32 cache's tile takes six times the matrix work of a 16-bit one, so
+//   splitting pays earlier: partitions of 128 keys on, the smallest that fits
+//   the slots, for tiles of more than one and a half of them (16 rows after
+//   1000 keys, 14/2 heads x 64: 18.2 us in 128-key partitions, 20.9 in 192, 22.2
+//   in 256, 36.5 on the 32-row tiles; 300 rows after nothing 16.2, 21.3, 21.3
+//   and 31.1; 512 after 1024 35.2, 35.3, 38.0 and 42.8; 4 x 200 after 300, 16/16
+//   heads, 28.5, 28.5, 24.4 and 78).
 // Steps with more rows than arrival counters keep the 32-row tiles: a step
 // that splits nothing there runs without a workspace.
 PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok) {
   PrefillCut c;
   const int group = cfg.q_heads / cfg.kv_heads, bs = cfg.block_size;
-  if (cfg.chunk_q_tile > 0 || cfg.chunk_partition_tokens > 0 || cfg.kv_dtype == LE_F32 ||
+  const bool f32 = cfg.kv_dtype == LE_F32;
+  if (cfg.chunk_q_tile > 0 || cfg.chunk_partition_tokens > 0 || (f32 && cfg.head_dim != 64) ||
       (cfg.flags & LE_PLAN_TWO_LAUNCHES) || (cfg.head_dim != 64 && cfg.head_dim != 128) || group < 1 || group > 8 ||
       n_tok * cfg.kv_heads > kArrivalCounters)
     return c;
@@ -200,7 +213,7 @@ PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n,
   int64_t keys = total_keys();
   if (tiles == 0) return c;
   c.on = true;
-  c.wide = cfg.head_dim == 64 && keys >= 1000 * kPrefillSlots;
+  c.wide = cfg.head_dim == 64 && !f32 && keys >= 1000 * kPrefillSlots;
   c.rows = le::prefill_rows(c.wide, group);
   if (!c.wide) keys = total_keys();
   if (tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
@@ -215,8 +228,25 @@ PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n,
     c.bytes = rows * cfg.q_heads * (cfg.head_dim * 4 + 8);
     return (items * padded + tiles - 1) / tiles * cfg.kv_heads;
   };
-  c.part = kSmallPrefillPart;
-  if (workgroups() <= kSmallPrefill && c.bytes <= kSmallPrefillScratch) return c;
+  int64_t decode_bytes = 0;  // the decode rows' partials
+  for (int i = 0; i < n; i++)
+    if (s[i].len == 1) {
+      const int64_t pt = cfg.partition_tokens > 0 ? cfg.partition_tokens : kMixedPrefillPartition;
+      if (s[i].start >= pt) decode_bytes += (s[i].start / pt + 1) * cfg.q_heads * (cfg.head_dim * 4 + 8);
+    }
+  auto fits = [&](int64_t slots, int64_t scratch) {
+    return workgroups() <= slots && c.bytes <= scratch && c.bytes + decode_bytes <= kFinerPrefillScratch;
+  };
+  if (f32) {
+    for (c.part = kF32PrefillPart; c.part < kDefaultChunkPartition; c.part += 64) {
+      c.split_keys = c.part * 3 / 2;
+      if (fits(kPrefillSlots, kF32PrefillScratch)) return c;
+    }
+    c.split_keys = kPrefillSplitKeys;
+  } else {
+    c.part = kSmallPrefillPart;
+    if (fits(kSmallPrefill, kSmallPrefillScratch)) return c;
+  }
   c.part = std::max<int64_t>((keys / kPrefillSlots + 63) / 64 * 64, kDefaultChunkPartition);
   while (workgroups() > kPrefillSlots && c.part < longest * bs) c.part += (c.part / 8 + 63) / 64 * 64;
   return c;

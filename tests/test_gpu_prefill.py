@@ -1,4 +1,5 @@
-"""GPU parity of the prefill tiles (attention_prefill_wg.h) with the oracle at
+"""GPU parity of the prefill tiles (attention_prefill_wg.h, and
+attention_prefill_f32_wg.h for fp32 caches) with the oracle at
 the edges of their tiles, partitions and softmax base."""
 import numpy as np
 import pytest
@@ -92,3 +93,30 @@ def test_prefill_softmax_base(gpu, kind, hd):
         k[..., 0] = (-12.0 if kind == "negative" else pos[:, None] / 16)
     case.k_cache, case.v_cache = (oracle.f32_to_bf16(c) for c in (case.k_cache, case.v_cache))
     check(case, "f32", gpu)
+
+
+# fp32 caches of head_dim 64: every product to fp32 rounding. The bar is twice
+# the error of the 32-row tiles, which make the same roundings in another order,
+# and an ulp of the largest value for the order itself.
+@pytest.mark.parametrize("flags", [0, LE_PLAN_XCD_LOCAL])
+@pytest.mark.parametrize("heads,act,bs,split", [((14, 2, 64), "f32", 16, False), ((32, 4, 64), "bf16", 8, False),
+                                                ((3, 3, 64), "f32", 32, False), ((14, 2, 64), "f32", 16, True),
+                                                ((16, 16, 64), "f16", 64, True), ((8, 1, 64), "f32", 16, True)])
+def test_prefill_f32_tiles(gpu, heads, act, bs, split, flags):
+    H, KH, hd = heads
+    tile = 128 // (H // KH)
+    if split:
+        q_len, ctx = [5, 40, tile + 1, 3, 2, 1, 1], [193, 1500, 700, 3000, 385, 1100, 2500]
+    else:
+        q_len, ctx = [2, tile - 1, tile, min(tile + 1, 130), 65, 7, 3, 1, 1], [2, 63, 64, 130, 128, 65, 68, 40, 333]
+    ctx = [max(a, b) for a, b in zip(ctx, q_len)]
+    case = make_case(ctx, H, KH, hd, bs, q_len=q_len, seed=H + bs)
+    poison_unused(case)
+
+    def bar(qh, want):
+        old, _, plan = run_ragged(case, ACT[act], gpu, flags=flags, chunk_q_tile=32)
+        assert plan.plan.cfg.chunk_q_tile == 32
+        err = np.abs(old.astype(np.float64) - want) - OUT_REL[act] * np.abs(want)
+        return 2 * max(0.0, float(err.max())) + 2.0 ** -22 * float(np.nanmax(np.abs(case.v_cache)))
+
+    check(case, act, gpu, want_split=split, bar=bar, flags=flags)

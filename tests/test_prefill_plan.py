@@ -1,5 +1,5 @@
-"""How a step's chunk rows are cut into prefill tiles (16-bit caches, neither
-tile nor partition given): the work lists against the step, and against the
+"""How a step's chunk rows are cut into prefill tiles (16-bit caches, and fp32
+ones at head_dim 64; neither tile nor partition given): the work lists against the step, and against the
 32-row tiles of the same step (chunk_q_tile given), over head groups, block
 sizes, ragged rows, repeated sequences and step sizes."""
 import numpy as np
@@ -31,8 +31,11 @@ SHAPES = [(14, 2, 64), (32, 4, 64), (16, 16, 64), (32, 8, 128), (28, 4, 128), (6
 
 @pytest.mark.parametrize("heads", SHAPES)
 @pytest.mark.parametrize("bs", [8, 16, 64, 512])
-def test_prefill_tiles_cover_the_step(heads, bs):
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float32])
+def test_prefill_tiles_cover_the_step(heads, bs, kv):
     H, KH, hd = heads
+    if kv == torch.float32 and hd != 64:
+        pytest.skip("fp32 caches with head_dim 128 keep the 32-row tiles")
     rng = np.random.default_rng(H * 1000 + bs)
     wide = 0
     for n_chunks, max_rows, max_hist, n_decode in [(1, 2, 0, 0), (1, 40, 100, 3), (3, 300, 1500, 0), (2, 17, 9000, 5),
@@ -40,7 +43,7 @@ def test_prefill_tiles_cover_the_step(heads, bs):
         sl = step(rng, bs, n_chunks, max_rows, max_hist, n_decode)
 
         def make(**kw):
-            return kernels.Plan(sl, H, KH, hd, bs, torch.bfloat16, device="cpu", pin=False, **kw)
+            return kernels.Plan(sl, H, KH, hd, bs, kv, device="cpu", pin=False, **kw)
 
         plan, tiles32 = make(flags=LE_PLAN_XCD_LOCAL), make(flags=LE_PLAN_XCD_LOCAL, chunk_q_tile=32)
         P, old = plan.plan, tiles32.plan
@@ -49,6 +52,7 @@ def test_prefill_tiles_cover_the_step(heads, bs):
         wide += is_wide
         cols = 256 if is_wide else 128
         assert hd == 64 or not is_wide
+        assert kv == torch.bfloat16 or not is_wide
         pos, tables = plan.host_array("positions"), plan.host_array("tables")
         toff, items = plan.host_array("table_offset"), items_of(plan)
         stride = P.decode_ids_stride
@@ -84,15 +88,16 @@ def test_prefill_tiles_cover_the_step(heads, bs):
         owned += [int(d[5]) for d in dec if d[5] >= 0]
         assert sorted(owned) == list(range(P.n_parts))
         # scratch: no more than the 32-row tiles take, or a small step's bound
-        # (8 MiB for the tiles and 5 MB for finer decode partitions)
+        # (8 MiB for the tiles, 16 with an fp32 cache, and 5 MB for finer decode partitions)
         row_bytes = H * (hd * 4 + 8)
-        assert P.n_parts * row_bytes <= max(old.n_parts * row_bytes + 5_000_000, (8 << 20) + 5_000_000)
+        small = (16 if kv == torch.float32 else 8) << 20
+        assert P.n_parts * row_bytes <= max(old.n_parts * row_bytes, small) + 5_000_000
         assert P.n_parts * row_bytes <= max(old.n_parts * row_bytes, 31 << 20)
-    assert wide > 0 or heads != (32, 4, 64)  # both widths were seen
+    assert wide > 0 or heads != (32, 4, 64) or kv == torch.float32  # both widths were seen
 
 
 def test_prefill_tiles_only_where_asked_for_nothing():
-    """Explicit sizes, the two-launch flag, fp32 caches and steps without
+    """Explicit sizes, the two-launch flag, fp32 caches with head_dim 128 and steps without
     arrival counters for every row keep the 32-row tiles; a plan's own
     resolved configuration gives the same plan again."""
     sl = step(np.random.default_rng(1), 16, 2, 400, 900, 3)
@@ -106,7 +111,7 @@ def test_prefill_tiles_only_where_asked_for_nothing():
                  partition_tokens=auto.cfg.partition_tokens)
     assert (again.n_chunk_items, again.n_parts, again.bytes) == (auto.n_chunk_items, auto.n_parts, auto.bytes)
     for kw in (dict(chunk_q_tile=32), dict(chunk_q_tile=16), dict(chunk_partition_tokens=256),
-               dict(flags=LE_PLAN_TWO_LAUNCHES), dict(kv=torch.float32)):
+               dict(flags=LE_PLAN_TWO_LAUNCHES), dict(kv=torch.float32, heads=(32, 8, 128))):
         assert make(**kw).cfg.chunk_q_tile in (16, 32)
     many = [kernels.Slice(i, 0, 600, True, np.arange(38, dtype=np.int32), np.zeros(600, np.int32)) for i in range(7)]
     assert make(heads=(16, 16, 64), slices=many).cfg.chunk_q_tile == 32  # 4200 rows x 16 kv heads
