@@ -37,3 +37,34 @@ def test_argmax_ties_nans_and_empty_rows(gpu):
     x[7, 12345] = np.inf; x[7, 23456] = np.inf
     x[8, 4 * 777 + 1] = 30.0; x[8, 4 * 777 + 3] = 30.0  # tie inside one 16-byte piece
     _check(x)
+
+
+# edges of the groups of eight 16-byte pieces a thread reads at a time (32768
+# elements), elements past the last whole piece, rows at addresses that are not
+# a multiple of 16. Each row's winner, or its tied pair, sits at such an edge;
+# NaN and -inf rows among them.
+@pytest.mark.parametrize("rows,vocab", [(7, 1), (7, 3), (14, 5), (9, 4095), (14, 4097), (30, 32767), (30, 32768),
+                                        (30, 32769), (70, 65541), (5, 151937)])
+def test_argmax_piece_edges(gpu, rows, vocab):
+    rng = np.random.default_rng(rows + vocab)
+    x = rng.standard_normal((rows, vocab), dtype=np.float32)
+    ends = (0, 4, 4096, 8192, 32768, 65536, vocab // 4 * 4, vocab)
+    edges = sorted({e + d for e in ends for d in (-1, 0, 1) if 0 <= e + d < vocab})
+    for r in range(rows):
+        kind = r % 7
+        if kind == 0:
+            x[r, int(rng.choice(edges))] = 40.0
+        elif kind == 1:
+            x[r, rng.choice(edges, 2)] = 40.0
+        elif kind == 2:
+            x[r, vocab - 1] = 40.0
+        elif kind == 3:
+            x[r] = -np.inf if r % 2 else np.nan
+        elif kind == 4:
+            x[r, 0] = np.nan
+        elif kind == 5:
+            x[r, :-1] = np.nan
+            x[r, 0] = -np.inf
+        else:
+            x[r] = rng.integers(0, 2, vocab)
+    _check(x)
