@@ -34,6 +34,7 @@
 namespace {
 
 constexpr int kDefaultPartition = 640;       // decode rows: smallest automatic partition
+constexpr int kSmallStepPartF32 = 256;       // fp32 cache: the smallest in a step with a CU for every workgroup
 constexpr int kMaxAutoPartition = 4096;      // decode rows: largest automatic partition
 constexpr int kMixedStepPartition = 2048;    // decode rows beside chunk rows: smallest automatic partition
 constexpr int kPartitionQuantum = 128;       // 4 waves x 32-key fp32 tiles
@@ -356,6 +357,20 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
           if (slices[i].len == 1) n += std::min<int64_t>((slices[i].start / bs + 1 + pb - 1) / pb, max_parts);
         return n;
       };
+      // fp32 keys are twice the bytes: a step that leaves CUs without a
+      // workgroup takes shorter partitions, the shortest (two 32-key tiles a
+      // wave on) that still gives every workgroup a CU of its own, where the
+      // stream of a partition is the longest part (us a call, 640-key
+      // partitions and these: 48 rows of 32-2048 keys, 14/2 heads x 64, 16.9
+      // and 11.9; one row of 2000 14.3 and 10.8). A second workgroup on a CU
+      // slows the first: 64 rows of 64-4096, 256 against 328 workgroups, 19.3
+      // and 22.4.
+      if (cfg.kv_dtype == LE_F32)
+        for (int64_t pt = kSmallStepPartF32; pt < part; pt += kPartitionQuantum)
+          if (items_at(pt) * cfg.kv_heads <= kTargetItems / 2) {
+            part = pt;
+            break;
+          }
       while (part < kMaxAutoPartition && items_at(part) * cfg.kv_heads > kTargetItems) part += kPartitionQuantum;
     }
     cfg.partition_tokens = static_cast<int32_t>(std::min<int64_t>(part, kMaxAutoPartition));

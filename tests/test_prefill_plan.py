@@ -116,3 +116,29 @@ def test_prefill_tiles_only_where_asked_for_nothing():
     many = [kernels.Slice(i, 0, 600, True, np.arange(38, dtype=np.int32), np.zeros(600, np.int32)) for i in range(7)]
     assert make(heads=(16, 16, 64), slices=many).cfg.chunk_q_tile == 32  # 4200 rows x 16 kv heads
     assert make(heads=(16, 16, 64), slices=many[:6]).cfg.chunk_q_tile <= 0
+
+
+def test_fp32_decode_partitions_of_a_small_step():
+    """fp32 caches, decode rows only: the shortest partition from 256 keys on
+    that leaves at most one workgroup a CU; the 16-bit rule (640 keys and more)
+    where there is none."""
+    rng = np.random.default_rng(12)
+    seen = set()
+    for trial in range(60):
+        H, KH = [(14, 2), (32, 4), (32, 8), (16, 16)][trial % 4]
+        lens = rng.integers(1, int(rng.choice([300, 1400, 5000])), size=int(rng.integers(1, 100)))
+        sl = [kernels.Slice(i, int(n) - 1, 1, True, np.arange((n + 15) // 16, dtype=np.int32), np.zeros(int(n), np.int32))
+              for i, n in enumerate(lens)]
+
+        def make(kv):
+            return kernels.Plan(sl, H, KH, 64, 16, kv, device="cpu", pin=False).plan
+
+        def items(pt):
+            return sum(-(-int(n) // pt) for n in lens)
+
+        f32, b16 = make(torch.float32), make(torch.bfloat16)
+        fits = [pt for pt in range(256, b16.cfg.partition_tokens, 128) if items(pt) * KH <= 256]
+        assert f32.cfg.partition_tokens == (fits[0] if fits else b16.cfg.partition_tokens)
+        assert f32.n_decode_items == items(f32.cfg.partition_tokens)
+        seen.add(min(f32.cfg.partition_tokens, 640))
+    assert {256, 640} <= seen
