@@ -98,6 +98,7 @@ struct DecodeParams {
   int ids_stride;
   int n_rows;               // items, or tokens when items is null
   int nsplit;
+  int share_items, min_part;  // items null: workgroups per kv head that share the keys, least keys of a partition
   int q_heads, kv_heads, head_dim, block_size;
   float scale_log2;         // softmax scale * log2(e)
   int64_t num_cache_blocks;
@@ -161,5 +162,19 @@ hipError_t attention_ragged(const DecodeParams& d, const ChunkParams& c, int act
 // Split count for the reference-shaped entry point, where the host does not
 // know the context lengths: enough workgroups to cover the chip several times.
 int decode_nsplit(int n_tokens, int kv_heads);
+
+// How its rows are then cut on the device (resolve() in attention_decode_wg.h):
+// the step's keys shared by about this many workgroups, in partitions of at
+// least this many keys; rows = tokens x kv heads. Measured (us a call):
+// * 1024 workgroups against 512 below 512 rows: 33 rows of 3626 keys, fp32, 28/4
+//   heads x 128, 139 against 159 (four partitions a row just pass one round at
+//   two workgroups a CU); 40 of 663-5304, bf16, 8/8 x 128, 102 against 108; 24 of
+//   100-3000, fp16, 32/8 x 128, 39.7 against 39.8. From 512 rows on 512: 256 rows of
+//   64-2048, 14/2 x 64, 34.9 against 41.1.
+// * 512 keys against 256 from 128 rows on: 64 of 64-4096, 14/2 x 64, 20.5 against
+//   25.7. Below that, where CUs are idle, 256: 7 of 1-1674, bf16, 32/8 x 128, 10.9
+//   against 14.2; 48 of 32-2048, fp32, 14/2 x 64, 16.5 against 22.5.
+constexpr int unplanned_items(int64_t rows) { return rows < 512 ? 1024 : 512; }
+constexpr int unplanned_part(int64_t rows) { return rows < 128 ? 256 : 512; }
 
 }  // namespace le
