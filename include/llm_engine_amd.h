@@ -233,6 +233,12 @@ static inline const int32_t* le_plan_dev_array(const le_step_plan* plan, int64_t
  * absolute position against the cached prefix. Split rows are merged inside
  * their launch. The result equals le_attention_decode on the same step.
  * ------------------------------------------------------------------------ */
+/* Bytes of workspace that a packed step needs: 0 (a null workspace will do) if
+ * no row is split over partitions, which holds for every step with decode rows
+ * of at most 640 keys (2048 beside chunk rows, or the given partition) and chunk
+ * rows that end within 384. Otherwise it depends on how the step is cut, and a
+ * large step may need less than a small one (chunk rows that fill the chip are
+ * not split): size the buffer by the plan, not by the largest step. */
 size_t le_ragged_workspace_size(const le_step_plan* plan);
 
 int le_ragged_paged_attention(const void* q, le_dtype act_dtype, const void* k_cache,

@@ -146,8 +146,8 @@ struct PrefillCut {
   int64_t part = 0;
   int64_t split_keys = kPrefillSplitKeys;
   int64_t bytes = 0;  // at most this much for the tiles' partials
-  // Partitions (whole blocks) of a tile over nb key blocks of bs: with `part`
-  // at least kDefaultChunkPartition, never more than the 32-row tiles take.
+  // Partitions (whole blocks) of a tile over nb key blocks of bs; with `part` at
+  // least kDefaultChunkPartition, no more than a 32-row tile with that end takes.
   int parts(int64_t nb, int bs) const {
     if (part == 0 || nb * bs <= split_keys) return 1;
     const int64_t pb = std::max((part + bs - 1) / bs, (nb + kMaxChunkParts - 1) / kMaxChunkParts);
@@ -191,7 +191,9 @@ void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
 //   heads, 28.5, 28.5, 24.4 and 78).
 // Steps with more rows than arrival counters keep the 32-row tiles: a step
 // that splits nothing there runs without a workspace.
-PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok) {
+// A step that the plain cut does not split (may_split false) keeps its tiles
+// whole: it needs no workspace, and a caller may pass none.
+PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok, bool may_split) {
   PrefillCut c;
   const int group = cfg.q_heads / cfg.kv_heads, bs = cfg.block_size;
   const bool f32 = cfg.kv_dtype == LE_F32;
@@ -217,7 +219,7 @@ PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n,
   c.wide = cfg.head_dim == 64 && !f32 && keys >= 1000 * kPrefillSlots;
   c.rows = le::prefill_rows(c.wide, group);
   if (!c.wide) keys = total_keys();
-  if (tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
+  if (!may_split || tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
   const int64_t padded = cfg.kv_heads % kXcds == 0 ? tiles : (tiles + kXcds - 1) / kXcds * kXcds;
   auto workgroups = [&] {  // with partitions of c.part keys; sets c.bytes
     int64_t items = 0, rows = 0;
@@ -313,8 +315,20 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     max_pos = std::max(max_pos, last);
   }
   if (n_tok > INT32_MAX / 2) return LE_EUNSUPPORTED;
-  const PrefillCut pre = cut_prefill(asked, slices, n_slices, n_tok);
-  if (!fixed && cfg.partition_tokens <= 0) {
+  // ---- decode partitions ----
+  const bool auto_part = !fixed && cfg.partition_tokens <= 0;
+  bool chunk_rows = false;
+  for (int i = 0; i < n_slices; i++) chunk_rows |= slices[i].len > 1;
+  const int max_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
+  auto items_at = [&](int64_t pt) {  // decode items per kv head with partitions of pt keys
+    const int64_t pb = (pt + bs - 1) / bs;
+    int64_t n = 0;
+    for (int i = 0; i < n_slices; i++)
+      if (slices[i].len == 1) n += std::min<int64_t>((slices[i].start / bs + 1 + pb - 1) / pb, max_parts);
+    return n;
+  };
+  int64_t part = cfg.partition_tokens, shared = 0;  // shared: one workgroup's share of the step's keys
+  if (auto_part) {
     // Size decode partitions so the step has about kTargetItems workgroups,
     // two per CU. Each workgroup pays a fixed chain of dependent memory
     // round trips (block ids, then K/V; partial store, arrival counter, merge)
@@ -327,36 +341,44 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
       if (slices[i].len == 1)
         for (int r = 0; r < slices[i].len; r++) ctx += slices[i].start + r + 1;
     const int64_t per_kvh = std::max<int64_t>(1, kTargetItems / cfg.kv_heads);
-    int64_t part = (ctx + per_kvh - 1) / per_kvh;
-    part = (part + kPartitionQuantum - 1) / kPartitionQuantum * kPartitionQuantum;
-    part = std::max<int64_t>(part, kDefaultPartition);
-    // In a mixed step the chunk workgroups hold most CUs for the first half
-    // of the launch; splitting the decode rows further only adds merges
-    // (config 3: 22.7 us with the rule above, 22.4 us with 2048 tokens).
-    bool chunk_rows = false;
-    for (int i = 0; i < n_slices; i++) chunk_rows |= slices[i].len > 1;
+    shared = (ctx + per_kvh - 1) / per_kvh;
+    shared = (shared + kPartitionQuantum - 1) / kPartitionQuantum * kPartitionQuantum;
+    part = std::max<int64_t>(shared, kDefaultPartition);
     if (chunk_rows) {
-      // (beside prefill tiles, whose workgroups share a CU with the decode
-      // rows', 1024: 2 x 512 rows after 1024 keys and 32 decode rows 25.6
-      // against 31.1 us). Those partitions need at most 5 MB more of partials
-      // than 2048-key ones: where the tiles' own leave that much of the static
-      // scratch, else 2048 as before.
-      const bool finer = pre.on && pre.bytes <= kFinerPrefillScratch;
-      part = std::max<int64_t>(part, finer ? kMixedPrefillPartition : kMixedStepPartition);
+      // In a mixed step the chunk workgroups hold most CUs for the first half
+      // of the launch; splitting the decode rows further only adds merges
+      // (config 3 on 32-row tiles: 22.7 us with the rule above, 22.4 us with
+      // 2048 tokens).
+      part = std::max<int64_t>(part, kMixedStepPartition);
     } else {
       // The rows' partitions are whole ceilings, so the rule above can
       // overshoot: grow the partition until the step's workgroups fit one
       // round at two per CU (TinyLlama-shaped decode steps, 64 rows, 4 kv
       // heads: 136-144 items per kv head ran 20.6-21.5 us per launch, 120
       // items 15-16 us).
-      const int max_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
-      auto items_at = [&](int64_t pt) {
-        const int64_t pb = (pt + bs - 1) / bs;
-        int64_t n = 0;
-        for (int i = 0; i < n_slices; i++)
-          if (slices[i].len == 1) n += std::min<int64_t>((slices[i].start / bs + 1 + pb - 1) / pb, max_parts);
-        return n;
-      };
+      while (part < kMaxAutoPartition && items_at(part) * cfg.kv_heads > kTargetItems) part += kPartitionQuantum;
+    }
+    part = std::min<int64_t>(part, kMaxAutoPartition);
+  }
+  // The plain cut: these decode partitions, chunk rows over 384 keys. A step
+  // that it does not split needs no workspace and may be run without one, so
+  // the finer cuts below, which pay off on such steps too (32 decode rows of
+  // 1500 keys beside chunks, fp32 rows of 300-640 keys), are taken only where
+  // it splits something.
+  bool splits = false;
+  for (int i = 0; i < n_slices; i++)
+    splits |= (slices[i].start + slices[i].len - 1) / bs + 1 >
+              round_to_blocks(slices[i].len > 1 ? kDefaultChunkPartition : static_cast<int>(part), bs);
+  const PrefillCut pre = cut_prefill(asked, slices, n_slices, n_tok, splits);
+  if (auto_part) {
+    if (splits && chunk_rows && pre.on && pre.bytes <= kFinerPrefillScratch) {
+      // Beside prefill tiles, whose workgroups share a CU with the decode
+      // rows', 1024 keys: 2 x 512 rows after 1024 keys and 32 decode rows 25.6
+      // against 31.1 us. Those partitions need at most 5 MB more of partials
+      // than 2048-key ones: where the tiles' own leave that much of the static
+      // scratch, else 2048 as before.
+      part = std::min<int64_t>(std::max<int64_t>(shared, kMixedPrefillPartition), kMaxAutoPartition);
+    } else if (splits && !chunk_rows && cfg.kv_dtype == LE_F32) {
       // fp32 keys are twice the bytes: a step that leaves CUs without a
       // workgroup takes shorter partitions, the shortest (two 32-key tiles a
       // wave on) that still gives every workgroup a CU of its own, where the
@@ -365,24 +387,21 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
       // and 11.9; one row of 2000 14.3 and 10.8). A second workgroup on a CU
       // slows the first: 64 rows of 64-4096, 256 against 328 workgroups, 19.3
       // and 22.4.
-      if (cfg.kv_dtype == LE_F32)
-        for (int64_t pt = kSmallStepPartF32; pt < part; pt += kPartitionQuantum)
-          if (items_at(pt) * cfg.kv_heads <= kTargetItems / 2) {
-            part = pt;
-            break;
-          }
-      while (part < kMaxAutoPartition && items_at(part) * cfg.kv_heads > kTargetItems) part += kPartitionQuantum;
+      for (int64_t pt = kSmallStepPartF32; pt < part; pt += kPartitionQuantum)
+        if (items_at(pt) * cfg.kv_heads <= kTargetItems / 2) {
+          part = pt;
+          break;
+        }
     }
-    cfg.partition_tokens = static_cast<int32_t>(std::min<int64_t>(part, kMaxAutoPartition));
+    cfg.partition_tokens = static_cast<int32_t>(part);
   }
   const int dec_pb = round_to_blocks(cfg.partition_tokens, bs);
   const int chk_pb = round_to_blocks(cfg.chunk_partition_tokens, bs);
   const bool mfma_chunks = true;  // chunk rows on MFMA tiles, every cache type
-  const int max_decode_parts = std::max(1, kMaxMergeEntries / std::max(1, cfg.q_heads / cfg.kv_heads));
 
   // Fixed layout: every row owns parts_cap partial slots and every table
   // table_capacity entries, whatever its current length.
-  const int parts_cap = fixed ? std::min((cfg.table_capacity + dec_pb - 1) / dec_pb, max_decode_parts) : 0;
+  const int parts_cap = fixed ? std::min((cfg.table_capacity + dec_pb - 1) / dec_pb, max_parts) : 0;
   if (fixed) n_table = static_cast<int64_t>(n_seqs) * cfg.table_capacity;
 
   // Table offset of each distinct sequence in the concatenated tables.
@@ -434,7 +453,7 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
           const int pos = s.start + r;
           const int nb = pos / bs + 1;
           // Partitions per row are capped (the merging workgroup loads them all).
-          const int J = std::min((nb + dec_pb - 1) / dec_pb, max_decode_parts);
+          const int J = std::min((nb + dec_pb - 1) / dec_pb, max_parts);
           // Split rows are merged inside the decode launch by the last
           // partition to finish, so they need no combine item.
           for (int j = 0; j < J; j++) {

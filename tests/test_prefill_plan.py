@@ -138,7 +138,50 @@ def test_fp32_decode_partitions_of_a_small_step():
 
         f32, b16 = make(torch.float32), make(torch.bfloat16)
         fits = [pt for pt in range(256, b16.cfg.partition_tokens, 128) if items(pt) * KH <= 256]
+        if b16.n_parts == 0:  # a step that runs without a workspace keeps doing so
+            fits = []
         assert f32.cfg.partition_tokens == (fits[0] if fits else b16.cfg.partition_tokens)
         assert f32.n_decode_items == items(f32.cfg.partition_tokens)
         seen.add(min(f32.cfg.partition_tokens, 640))
     assert {256, 640} <= seen
+
+
+def plain_cut_splits(sl, H, KH, bs, partition=0):
+    """Whether the plain cut (32-row tiles over 384 keys; decode rows over 640 keys, 2048 beside chunk rows, and more
+    in steps of many keys) splits any row, that is, whether the step needs a workspace at all."""
+    decode = [s.start + 1 for s in sl if s.len == 1]
+    chunks = [s for s in sl if s.len > 1]
+    part = -(-sum(decode) // max(1, 512 // KH))
+    part = min(max(-(-part // 128) * 128, 2048 if chunks else 640), 4096) if partition == 0 else partition
+    if partition == 0 and not chunks:
+        while part < 4096 and sum(-(-n // part) for n in decode) * KH > 512:
+            part += 128
+    blocks = lambda n: -(-n // bs)
+    return any(blocks(n) > blocks(part) for n in decode) or any(blocks(s.start + s.len) > blocks(384) for s in chunks)
+
+
+@pytest.mark.parametrize("heads", SHAPES)
+@pytest.mark.parametrize("kv", [torch.bfloat16, torch.float16, torch.float32])
+def test_steps_without_workspace(heads, kv):
+    """A step whose plain cut splits nothing runs without a workspace (a null one included), whatever finer partitions
+    its cut could take: decode rows beside short chunks, fp32 prompts, fp32 decode rows."""
+    H, KH, hd = heads
+    rng = np.random.default_rng(H + KH)
+    seen = {True: 0, False: 0}
+    for trial in range(120):
+        bs = int(rng.choice([8, 16, 32, 64, 512]))
+        n_chunks, n_decode = int(rng.integers(0, 5)), int(rng.integers(0, 30))
+        max_rows, max_hist = int(rng.choice([10, 130, 380, 500])), int(rng.choice([0, 100, 600, 2040, 2500]))
+        if n_chunks + n_decode == 0:
+            continue
+        sl = step(rng, bs, n_chunks, max_rows, max_hist, n_decode)
+        for s in sl[:n_chunks]:  # chunks mostly within the plain cut's partition
+            if trial % 3 and s.start + s.len > 384:
+                s.start = max(0, 384 - s.len)
+                s.blocks = s.blocks[:(s.start + s.len + bs - 1) // bs]
+        partition = int(rng.choice([0, 0, 640, 2048]))
+        plan = kernels.Plan(sl, H, KH, hd, bs, kv, device="cpu", pin=False, partition_tokens=partition)
+        splits = plain_cut_splits(sl, H, KH, bs, partition)
+        assert splits or plan.workspace_size() == 0, (trial, plan.plan.n_parts, [(s.start, s.len) for s in sl])
+        seen[splits] += 1
+    assert min(seen.values()) > 15
