@@ -201,7 +201,8 @@ typedef struct le_step_plan {
       off_table_offset, off_cu_seqlens_q, off_seq_lens_k, off_logit_rows, off_decode_items,
       off_chunk_items, off_combine_items;
   int64_t off_decode_ids;     /* block ids of each decode item, then of each chunk item,
-                                 decode_ids_stride apart */
+                                 decode_ids_stride apart (a tile with more than 128, and than
+                                 every decode item, reads the tables: its row is empty) */
   int32_t decode_ids_stride;  /* entries per work item in that array (padded with -1) */
   int32_t xcd_local;          /* 1: every split row's or tile's partitions sit at item indices
                                  equal modulo 8 (LE_PLAN_XCD_LOCAL honoured) */

@@ -67,7 +67,7 @@ __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32S
   const int bs_mask = p.block_size - 1;
   const int64_t row_bytes = static_cast<int64_t>(p.kv_heads) * HD * 4;
   const int key_begin = it.blk_begin << bs_shift;
-  const int32_t* ids = p.item_ids + static_cast<int64_t>(item) * p.ids_stride;
+  const int32_t* ids = tile_ids(p, it, item);
   const char* kbase = static_cast<const char*>(p.k_cache) + kvh * (HD * 4);
   const char* vbase = static_cast<const char*>(p.v_cache) + kvh * (HD * 4);
 

@@ -197,6 +197,11 @@ __device__ __forceinline__ void finish_tile(const ChunkParams& p, const ChunkIte
   if (tid == 0) __hip_atomic_store(counter, arrival_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The item's block ids: the plan's list, or, past its width, the sequence's table.
+__device__ __forceinline__ const int32_t* tile_ids(const ChunkParams& p, const ChunkItem& it, int item) {
+  return it.seq < 0 ? p.tables + ~it.seq + it.blk_begin : p.item_ids + static_cast<int64_t>(item) * p.ids_stride;
+}
+
 // One prefill workgroup: item `item`, kv head `kvh`, NC column tiles a wave.
 template <typename ACT, typename KV, int HD, int NC>
 __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>& sm, int item, int kvh) {
@@ -225,7 +230,7 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
   const int bs_mask = p.block_size - 1;
   const int64_t row_bytes = static_cast<int64_t>(p.kv_heads) * HD * 2;
   const int key_begin = it.blk_begin << bs_shift;
-  const int32_t* ids = p.item_ids + static_cast<int64_t>(item) * p.ids_stride;
+  const int32_t* ids = tile_ids(p, it, item);
   const char* kbase = static_cast<const char*>(p.k_cache) + kvh * (HD * 2);
   const char* vbase = static_cast<const char*>(p.v_cache) + kvh * (HD * 2);
 

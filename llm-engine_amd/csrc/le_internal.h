@@ -28,12 +28,15 @@ struct DecodeItem {
 };
 
 // Chunk work item: query rows [tok_begin, tok_begin + n_q) (consecutive
-// positions of one sequence, at most 32) over key blocks [blk_begin, blk_end)
+// positions of one sequence, at most 32, or prefill_rows() of a prefill tile)
+// over key blocks [blk_begin, blk_end)
 // of its table, partition `part` of the tile's part_stride partitions. Row
 // tok_begin + i writes partial part0 + i * part_stride, or, when part0 < 0,
 // its normalised output directly; the last partition of the tile to arrive
 // (per kv head) merges partials [part0 - part + i * part_stride, ... +
 // part_stride) of each row.
+// seq is the sequence's index, or, of a prefill tile with more block ids than
+// are listed with the item, ~ where its table starts.
 struct ChunkItem {
   int32_t tok_begin, n_q, blk_begin, blk_end, part0, part_stride, seq, part;
   // keys of [blk_begin * block_size, ...) that hold a live position (at most
@@ -131,7 +134,8 @@ struct ChunkParams {
   void* out;
   PartialLayout parts;
   const ChunkItem* items;
-  const int32_t* item_ids;  // block ids of item i at item_ids[i * ids_stride + j]
+  // block ids of item i at item_ids[i * ids_stride + j] (its seq < 0: in the tables)
+  const int32_t* item_ids;
   int ids_stride;
   int n_items;
   int q_heads, kv_heads, head_dim, block_size;
@@ -143,8 +147,7 @@ struct ChunkParams {
 hipError_t attention_chunk(const ChunkParams& p, int act_dtype, int kv_dtype, hipStream_t stream);
 
 // Chunk rows as prefill tiles (attention_prefill.hip; 16-bit caches and fp32 ones of head_dim 64): an item
-// holds prefill_rows() consecutive rows, its block ids are read from the
-// step's tables. A plan whose chunk items are such tiles leaves
+// holds prefill_rows() consecutive rows. A plan whose chunk items are such tiles leaves
 // cfg.chunk_q_tile at kPrefillTiles or kWidePrefillTiles (an explicit row tile
 // is 16 or 32; as an input, both mean the default).
 constexpr int kPrefillTiles = 0, kWidePrefillTiles = -1;

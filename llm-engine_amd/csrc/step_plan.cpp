@@ -58,6 +58,7 @@ constexpr int kF32PrefillPart = 128;         // smallest partition of an fp32 pr
 constexpr int64_t kF32PrefillScratch = 16 << 20;    // the same with an fp32 cache
 constexpr int64_t kFinerPrefillScratch = 24 << 20;  // bytes of the tiles' partials up to which decode rows split finer
 constexpr int64_t kArrivalCounters = 65536;  // (row, kv head) arrival counters of a workspace
+constexpr int kTileListIds = 128;            // block ids of a prefill tile that are listed beside the decode items
 constexpr int kXcds = 8;                     // MI355X: XCDs, each with its own L2
 constexpr int kItemOverheadBlocks = 8;       // a decode item's fixed cost, in streamed blocks    // block ids of one chunk item the kernel stages
 
@@ -553,10 +554,19 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
   P.off_combine_items = take(0);
   // Each work item's block ids at a fixed stride (decode items, then chunk
   // items), so a workgroup can fetch them in the same memory round trip as
-  // its item.
+  // its item. A prefill tile may hold the whole of a long context and would
+  // widen every item's row, past what a decode workgroup takes ahead of its
+  // item (64 rows of 1024 keys beside a chunk after 16384, block size 8: 128 ids
+  // against 2304): one with more ids than the decode items and kTileListIds
+  // reads the step's tables instead (seq: ~ where its table starts), which
+  // costs it nothing, as its loads wait for the item anyway.
   int32_t ids_stride = 0;
   for (const auto& d : dec) ids_stride = std::max(ids_stride, d.blk_end - d.blk_begin);
-  for (const auto& c : chk) ids_stride = std::max(ids_stride, c.blk_end - c.blk_begin);
+  const int32_t listed = std::max(ids_stride, kTileListIds);
+  for (auto& c : chk) {
+    if (pre.on && c.blk_end - c.blk_begin > listed) c.seq = ~seq_table_off[c.seq];
+    else ids_stride = std::max(ids_stride, c.blk_end - c.blk_begin);
+  }
   if (fixed) ids_stride = std::max(dec_pb, (cfg.table_capacity + parts_cap - 1) / parts_cap);
   ids_stride = (ids_stride + 3) / 4 * 4;
   P.decode_ids_stride = ids_stride;
@@ -624,10 +634,10 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     int32_t* ids = arr(P.off_decode_ids) + dec.size() * static_cast<size_t>(ids_stride);
     for (size_t k = 0; k < chk.size(); k++) {
       const le::ChunkItem& c = chk[k];
-      const int32_t toff = table_offset[c.seq];
+      const int n = c.seq < 0 ? 0 : c.blk_end - c.blk_begin;
+      const int32_t* from = tables + (c.seq < 0 ? 0 : table_offset[c.seq]) + c.blk_begin;
       int32_t* row = ids + k * static_cast<size_t>(ids_stride);
-      for (int j = 0; j < ids_stride; j++)
-        row[j] = j < c.blk_end - c.blk_begin ? tables[toff + c.blk_begin + j] : -1;
+      for (int j = 0; j < ids_stride; j++) row[j] = j < n ? from[j] : -1;
     }
   }
   *plan = P;

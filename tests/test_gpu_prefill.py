@@ -60,6 +60,25 @@ def test_prefill_split_tiles(gpu, heads, kv, flags):
     check(case, "f32", gpu, want_split=True, flags=flags)
 
 
+# partitions of more than 128 blocks (of 8 keys): the tile reads its ids from
+# the step's tables, in a step with decode rows and without
+@pytest.mark.parametrize("decode", [False, True])
+@pytest.mark.parametrize("kv", ["bf16", "f32"])
+def test_prefill_ids_from_the_tables(gpu, kv, decode):
+    ctx, q_len = [17600, 300] + [700, 30] * decode, [21, 40] + [1, 1] * decode
+    case = make_case(ctx, 14, 2, 64, 8, q_len=q_len, seed=8, kv_bf16=kv == "bf16")
+    plan = run_ragged(case, torch.float32, gpu)[2]
+    P = plan.plan
+    items = plan.host.numpy()[P.off_chunk_items:][:36 * P.n_chunk_items].view(np.int32).reshape(-1, 9)
+    assert (items[:, 6] < 0).any() and (items[items[:, 1] > 0, 6] >= 0).any()
+
+    def bar(qh, want):  # twice the error of the 32-row tiles, which make the same roundings, and an ulp
+        old = run_ragged(case, torch.float32, gpu, chunk_q_tile=32)[0]
+        return 2 * max_abs(old, want) + 2.0 ** -22 * float(np.nanmax(np.abs(want)))
+
+    check(case, "f32", gpu, want_split=True, bar=bar)
+
+
 def test_prefill_wide_tiles(gpu):
     """256-column tiles: a step past 1000 keys per workgroup slot. The bar is
     twice the error of the 32-row tiles, which make the same roundings."""

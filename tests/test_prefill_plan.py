@@ -58,6 +58,8 @@ def test_prefill_tiles_cover_the_step(heads, bs, kv):
         stride = P.decode_ids_stride
         n_ids = P.n_decode_items + P.n_chunk_items
         ids = plan.host.numpy()[P.off_decode_ids:P.off_decode_ids + 4 * n_ids * stride].view(np.int32).reshape(-1, stride)
+        dec = plan.host.numpy()[P.off_decode_items:P.off_decode_items + 32 * P.n_decode_items].view(np.int32).reshape(-1, 8)
+        dec_ids = max((int(d[4] - d[3]) for d in dec), default=0)
         by_tile, owned, bins = {}, [], {}
         for k, it in enumerate(items):
             tb, nq, b0, b1, p0, J, seq, part, live = (int(x) for x in it)
@@ -65,8 +67,11 @@ def test_prefill_tiles_cover_the_step(heads, bs, kv):
                 continue
             assert 1 <= nq * (H // KH) <= cols and (np.diff(pos[tb:tb + nq]) == 1).all()
             assert b1 > b0 and live == min((b1 - b0) * bs, pos[tb + nq - 1] + 1 - b0 * bs) and live >= 1
-            row = ids[P.n_decode_items + k]
-            assert (row[:b1 - b0] == tables[toff[seq] + b0:toff[seq] + b1]).all() and (row[b1 - b0:] == -1).all()
+            row, n_ids, off = ids[P.n_decode_items + k], b1 - b0, toff[plan.host_array("token_seq")[tb]]
+            if seq < 0:  # too many ids to list: the kernel reads them at tables + ~seq + b0
+                assert ~seq == off and off + b1 <= P.n_table and n_ids > max(128, dec_ids)
+                n_ids = 0
+            assert (row[:n_ids] == tables[off + b0:off + b0 + n_ids]).all() and (row[n_ids:] == -1).all()
             by_tile.setdefault(tb, []).append((b0, b1, p0, J, part, nq))
             if J > 1:
                 owned += [p0 + r * J for r in range(nq)]
@@ -84,7 +89,6 @@ def test_prefill_tiles_cover_the_step(heads, bs, kv):
             rows |= set(range(tb, tb + nq))
         chunk_rows = sum(s.len for s in sl if s.len > 1)
         assert rows == set(range(chunk_rows))  # chunks first in these steps
-        dec = plan.host.numpy()[P.off_decode_items:P.off_decode_items + 32 * P.n_decode_items].view(np.int32).reshape(-1, 8)
         owned += [int(d[5]) for d in dec if d[5] >= 0]
         assert sorted(owned) == list(range(P.n_parts))
         # scratch: no more than the 32-row tiles take, or a small step's bound
@@ -185,3 +189,26 @@ def test_steps_without_workspace(heads, kv):
         assert splits or plan.workspace_size() == 0, (trial, plan.plan.n_parts, [(s.start, s.len) for s in sl])
         seen[splits] += 1
     assert min(seen.values()) > 15
+
+
+@pytest.mark.parametrize("bs", [8, 16])
+@pytest.mark.parametrize("hist", [0, 2000, 16384])
+def test_decode_ids_beside_prefill_tiles(bs, hist):
+    """The decode items' block ids in a mixed step stay as many as the decode rows need, or 128, whatever the chunk's
+    history: a tile over the whole of a long context does not widen their rows."""
+    def plan(chunk):
+        sl = [kernels.Slice(0, hist, 2048, True, np.arange((hist + 2048) // bs, dtype=np.int32),
+                            np.zeros(hist + 2048, np.int32))] if chunk else []
+        sl += [kernels.Slice(1 + i, 1023, 1, True, np.arange(1024 // bs, dtype=np.int32) + 7 * i,
+                             np.zeros(1024, np.int32)) for i in range(64)]
+        return kernels.Plan(sl, 32, 8, 128, bs, torch.bfloat16, device="cpu", pin=False, partition_tokens=1024)
+
+    def ids(p):
+        w = p.plan.decode_ids_stride
+        return p.host.numpy()[p.plan.off_decode_ids:][:64 * 4 * w].view(np.int32).reshape(64, w)
+
+    mixed, alone = plan(True), plan(False)
+    P, n = mixed.plan, 1024 // bs
+    assert P.cfg.chunk_q_tile == 0 and P.n_decode_items == alone.plan.n_decode_items == 64
+    assert alone.plan.decode_ids_stride == n and P.decode_ids_stride <= max(n, 128)
+    assert (ids(mixed)[:, :n] == ids(alone)).all() and (ids(mixed)[:, n:] == -1).all()
