@@ -153,8 +153,10 @@ typedef struct le_plan_config {
   int32_t chunk_q_tile;        /* query rows per chunk tile (16 or 32); 0 (or less) = default: 32
                                   with an fp32 cache of head_dim 128, else tiles of 128 or 256 query columns
                                   (row, head), sized and partitioned by the step; a packed plan's
-                                  cfg then holds 0 or -1 here and 0 below */
-  int32_t chunk_partition_tokens; /* key partition of chunk tiles; 0 = default */
+                                  cfg then holds 0 or -1 here and 0 (or -1) below */
+  int32_t chunk_partition_tokens; /* key partition of chunk tiles; 0 (or less) = default; -1 in a
+                                  packed plan's cfg: split rows may also run whole
+                                  (le_ragged_workspace_size) */
   int32_t flags;               /* LE_PLAN_* bits below; 0 = the defaults */
   int32_t table_capacity;      /* 0: tables packed exactly. > 0: a fixed layout for a step of
                                   decode rows only, so launches captured in a HIP graph can be
@@ -234,12 +236,13 @@ static inline const int32_t* le_plan_dev_array(const le_step_plan* plan, int64_t
  * absolute position against the cached prefix. Split rows are merged inside
  * their launch. The result equals le_attention_decode on the same step.
  * ------------------------------------------------------------------------ */
-/* Bytes of workspace that a packed step needs: 0 (a null workspace will do) if
- * no row is split over partitions, which holds for every step with decode rows
- * of at most 640 keys (2048 beside chunk rows, or the given partition) and chunk
- * rows that end within 384. Otherwise it depends on how the step is cut, and a
- * large step may need less than a small one (chunk rows that fill the chip are
- * not split): size the buffer by the plan, not by the largest step. */
+/* Bytes of workspace that a packed step needs. They depend on how it is cut, and
+ * a large step may need less than a small one (chunk rows that fill the chip are
+ * not split): size the buffer by the plan, not by the largest step. Outside the
+ * fixed layout, a step with decode rows of at most 640 keys (2048 beside chunk
+ * rows, or the given partition) and chunk rows that end within 384 also runs
+ * without a workspace (null, or too small): its rows then run whole, slower
+ * where the plan splits them. Other steps return LE_ENOSPACE then. */
 size_t le_ragged_workspace_size(const le_step_plan* plan);
 
 int le_ragged_paged_attention(const void* q, le_dtype act_dtype, const void* k_cache,

@@ -210,12 +210,16 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
     return LE_EINVAL;
   const size_t need = le_ragged_workspace_size(plan);
   if (need > 0 && !counters_fit(plan->n_tokens, cfg.kv_heads)) return LE_EUNSUPPORTED;
-  if (need > 0 && (!workspace || workspace_bytes < need)) return LE_ENOSPACE;
+  const bool short_ws = need > 0 && (!workspace || workspace_bytes < need);
+  // A step that the planner split only because that is faster runs whole
+  // without a workspace.
+  const bool whole = short_ws && cfg.chunk_partition_tokens == le::kMayRunWhole;
+  if (short_ws && !whole) return LE_ENOSPACE;
 
   const char* dev = static_cast<const char*>(plan->dev);
   auto arr = [&](int64_t off) { return reinterpret_cast<const int32_t*>(dev + off); };
   le::PartialLayout parts{};
-  if (need > 0)
+  if (need > 0 && !whole)
     parts = carve_partials(workspace, plan->n_parts, plan->n_tokens, cfg.q_heads, cfg.kv_heads,
                            cfg.head_dim);
   const float scale_log2 = scale * 1.4426950408889634f;
@@ -226,12 +230,12 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
   d.token_seq = arr(plan->off_token_seq); d.token_pos = arr(plan->off_positions);
   d.out = out; d.parts = parts;
   d.items = reinterpret_cast<const le::DecodeItem*>(dev + plan->off_decode_items);
-  d.item_ids = arr(plan->off_decode_ids);
+  d.item_ids = whole ? nullptr : arr(plan->off_decode_ids);
   d.ids_stride = plan->decode_ids_stride;
   d.n_rows = plan->n_decode_items; d.nsplit = 1;
   d.q_heads = cfg.q_heads; d.kv_heads = cfg.kv_heads; d.head_dim = cfg.head_dim;
   d.block_size = cfg.block_size; d.scale_log2 = scale_log2; d.num_cache_blocks = num_cache_blocks;
-  d.l2_local = plan->xcd_local && plan->n_parts > 0 && le::xcd_placement_holds(stream);
+  d.l2_local = plan->xcd_local && plan->n_parts > 0 && !whole && le::xcd_placement_holds(stream);
   // fixed-layout plans hold empty slots, so their item count says nothing
   // about the rounds
   d.wide = cfg.table_capacity == 0 && static_cast<int64_t>(plan->n_decode_items) * cfg.kv_heads >= 512;
@@ -257,6 +261,10 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
     }
   }
   if (rope && !d.k_new) return LE_EINVAL;  // q rows in QKV form need the in-launch path
+  if (whole && plan->n_chunk_items == 0) {  // the rows by token, one workgroup a row and kv head
+    d.items = nullptr;
+    d.n_rows = plan->n_tokens;
+  }
   if (plan->n_chunk_items == 0)
     return hip_status(le::attention_decode(d, act_dtype, kv_dtype, stream));
 
@@ -266,7 +274,7 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
   c.out = out; c.parts = parts;
   c.items = reinterpret_cast<const le::ChunkItem*>(dev + plan->off_chunk_items);
   // chunk items' block ids follow the decode items' at the same stride
-  c.item_ids = d.item_ids + static_cast<int64_t>(plan->n_decode_items) * plan->decode_ids_stride;
+  if (!whole) c.item_ids = d.item_ids + static_cast<int64_t>(plan->n_decode_items) * plan->decode_ids_stride;
   c.ids_stride = plan->decode_ids_stride;
   c.n_items = plan->n_chunk_items;
   c.q_heads = cfg.q_heads; c.kv_heads = cfg.kv_heads; c.head_dim = cfg.head_dim;
@@ -278,6 +286,11 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
   const bool two_launches = (cfg.flags & LE_PLAN_TWO_LAUNCHES) != 0;
   if (cfg.chunk_q_tile <= 0) {  // chunk items are prefill tiles
     const bool wide = cfg.chunk_q_tile == le::kWidePrefillTiles;
+    if (whole) {
+      e = le::attention_decode(d, act_dtype, kv_dtype, stream);
+      if (e != hipSuccess) return hip_status(e);
+      return hip_status(le::attention_prefill(c, wide, act_dtype, kv_dtype, stream));
+    }
     return hip_status(plan->n_decode_items > 0
                           ? le::attention_ragged_prefill(d, c, wide, act_dtype, kv_dtype, stream)
                           : le::attention_prefill(c, wide, act_dtype, kv_dtype, stream));

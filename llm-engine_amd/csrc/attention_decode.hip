@@ -12,7 +12,7 @@ namespace {
 constexpr int kMfmaWaves = 4;  // 8 waves measured slower (17.9 against 17.2 us)
 constexpr int kMfmaThreads = kMfmaWaves * 64;
 
-// Three instantiations of one workgroup body, by the registers they may use
+// Instantiations of one workgroup body, by the registers they may use
 // and the rows they take:
 // * mfma_kernel: two waves per SIMD (two workgroups per CU, at most 256
 //   registers a lane; 232 VGPRs, no spill). Launches of fewer than 512
@@ -43,11 +43,22 @@ __global__ __launch_bounds__(kMfmaThreads) void mfma_kernel_wide(DecodeParams p)
   dec::decode_wg<ACT, KV, HD, kMfmaWaves>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
+// The decode rows of a mixed step without a workspace (decode_wg's kWhole).
+template <typename ACT, typename KV, int HD>
+__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2))) void mfma_kernel_whole(DecodeParams p) {
+  __shared__ dec::DecodeSmem<KV, HD, kMfmaWaves> sm;
+  dec::decode_wg<ACT, KV, HD, kMfmaWaves, false, true>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
 template <typename ACT, typename KV>
 hipError_t launch(const DecodeParams& p, hipStream_t s) {
   const dim3 grid(p.n_rows, p.kv_heads, p.items ? 1 : p.nsplit);
   const bool wide = p.wide != 0;
-  if (p.rms_x && p.rope_max_pos > 0) {
+  if (p.items && !p.item_ids) {
+    if (p.k_new) return hipErrorInvalidValue;  // a mixed step has stored its rows
+    if (p.head_dim == 64) mfma_kernel_whole<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);
+    else mfma_kernel_whole<ACT, KV, 128><<<grid, kMfmaThreads, 0, s>>>(p);
+  } else if (p.rms_x && p.rope_max_pos > 0) {
     if (p.head_dim == 64) mfma_kernel_fold<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);
     else mfma_kernel_fold<ACT, KV, 128><<<grid, kMfmaThreads, 0, s>>>(p);
   } else if (p.head_dim == 64) {

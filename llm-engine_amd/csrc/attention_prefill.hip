@@ -13,13 +13,13 @@ __global__ __launch_bounds__(pre::kThreads, 2) void prefill_kernel(ChunkParams p
   __shared__ pre::PrefillSmem<HD> sm;
   // kv heads innermost: with 8 (4, 2) of them an XCD serves one (of one, of
   // two) head's K/V, whose rows its L2 then holds for all tiles of a sequence
-  pre::prefill_wg<ACT, KV, HD, NC>(p, sm, blockIdx.x / p.kv_heads, blockIdx.x % p.kv_heads);
+  pre::prefill_wg<ACT, KV, HD, NC, true>(p, sm, blockIdx.x / p.kv_heads, blockIdx.x % p.kv_heads);
 }
 
 template <typename ACT, int HD>
 __global__ __launch_bounds__(pre::kThreads, 2) void prefill_f32_kernel(ChunkParams p) {
   __shared__ pre::PrefillF32Smem<HD> sm;
-  pre::prefill_f32_wg<ACT, HD>(p, sm, blockIdx.x / p.kv_heads, blockIdx.x % p.kv_heads);
+  pre::prefill_f32_wg<ACT, HD, true>(p, sm, blockIdx.x / p.kv_heads, blockIdx.x % p.kv_heads);
 }
 
 }  // namespace

@@ -42,7 +42,7 @@ template <int HD> struct PrefillF32Smem {
 };
 
 // One prefill workgroup of an fp32 cache: item `item`, kv head `kvh`.
-template <typename ACT, int HD>
+template <typename ACT, int HD, bool kWhole = false>
 __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32Smem<HD>& sm, int item, int kvh) {
   using M = mma16<bf16_t>;
   using V8 = typename M::v8;
@@ -57,8 +57,8 @@ __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32S
   constexpr int U = kTileKeys / 32;
 
   char* lds = sm.lds;
-  const ChunkItem it = p.items[item];
-  if (it.n_q <= 0) return;  // padding that keeps split tiles on one XCD
+  const ChunkItem it = tile_item<kWhole>(p, item);
+  if (it.n_q <= 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;

@@ -197,13 +197,28 @@ __device__ __forceinline__ void finish_tile(const ChunkParams& p, const ChunkIte
   if (tid == 0) __hip_atomic_store(counter, arrival_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// The workgroup's item; n_q 0: nothing to do (padding that keeps split tiles
+// on one XCD, or a partition past the first of a tile that runs whole). kWhole:
+// without a list of ids there is no workspace, and split tiles run whole.
+template <bool kWhole> __device__ __forceinline__ ChunkItem tile_item(const ChunkParams& p, int item) {
+  ChunkItem it = p.items[item];
+  if (kWhole && !p.item_ids && it.n_q > 0) {
+    it.n_q = it.part == 0 ? it.n_q : 0;
+    it.part0 = -1;
+    it.key_live = p.token_pos[it.tok_begin] + it.n_q;
+    if (it.seq >= 0) it.seq = ~p.table_offset[it.seq];
+  }
+  return it;
+}
+
 // The item's block ids: the plan's list, or, past its width, the sequence's table.
 __device__ __forceinline__ const int32_t* tile_ids(const ChunkParams& p, const ChunkItem& it, int item) {
   return it.seq < 0 ? p.tables + ~it.seq + it.blk_begin : p.item_ids + static_cast<int64_t>(item) * p.ids_stride;
 }
 
 // One prefill workgroup: item `item`, kv head `kvh`, NC column tiles a wave.
-template <typename ACT, typename KV, int HD, int NC>
+// kWhole: p.item_ids may be null (tile_item).
+template <typename ACT, typename KV, int HD, int NC, bool kWhole = false>
 __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>& sm, int item, int kvh) {
   using M = mma16<KV>;
   using V8 = typename M::v8;
@@ -220,8 +235,8 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
 
   char* lds = sm.lds;
   int& last = sm.last;
-  const ChunkItem it = p.items[item];
-  if (it.n_q <= 0) return;  // padding that keeps split tiles on one XCD
+  const ChunkItem it = tile_item<kWhole>(p, item);
+  if (it.n_q <= 0) return;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;

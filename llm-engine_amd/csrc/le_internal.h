@@ -97,7 +97,10 @@ struct DecodeParams {
   int rms_hidden;
   float rms_eps;
   const DecodeItem* items;  // null: one item per (token, split) with `nsplit` splits
-  const int32_t* item_ids;  // with items: block ids of item i at item_ids[i * ids_stride + j]
+  // With items: block ids of item i at item_ids[i * ids_stride + j]. Null: a
+  // mixed step without a workspace; the first item of each row takes the whole
+  // row, the others leave.
+  const int32_t* item_ids;
   int ids_stride;
   int n_rows;               // items, or tokens when items is null
   int nsplit;
@@ -134,7 +137,9 @@ struct ChunkParams {
   void* out;
   PartialLayout parts;
   const ChunkItem* items;
-  // block ids of item i at item_ids[i * ids_stride + j] (its seq < 0: in the tables)
+  // block ids of item i at item_ids[i * ids_stride + j] (its seq < 0: in the
+  // tables). Null (prefill tiles): no workspace; the first item of each tile
+  // takes the whole tile, the others leave.
   const int32_t* item_ids;
   int ids_stride;
   int n_items;
@@ -143,6 +148,10 @@ struct ChunkParams {
   int64_t num_cache_blocks;
   int l2_local;  // split tiles' partitions share an XCD: partials through its L2 (as DecodeParams)
 };
+
+// cfg.chunk_partition_tokens of a plan whose split rows and tiles may run
+// whole, for a caller without a workspace (as an input, the default).
+constexpr int kMayRunWhole = -1;
 
 hipError_t attention_chunk(const ChunkParams& p, int act_dtype, int kv_dtype, hipStream_t stream);
 

@@ -192,9 +192,7 @@ void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
 //   heads, 28.5, 28.5, 24.4 and 78).
 // Steps with more rows than arrival counters keep the 32-row tiles: a step
 // that splits nothing there runs without a workspace.
-// A step that the plain cut does not split (may_split false) keeps its tiles
-// whole: it needs no workspace, and a caller may pass none.
-PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok, bool may_split) {
+PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok) {
   PrefillCut c;
   const int group = cfg.q_heads / cfg.kv_heads, bs = cfg.block_size;
   const bool f32 = cfg.kv_dtype == LE_F32;
@@ -220,7 +218,7 @@ PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n,
   c.wide = cfg.head_dim == 64 && !f32 && keys >= 1000 * kPrefillSlots;
   c.rows = le::prefill_rows(c.wide, group);
   if (!c.wide) keys = total_keys();
-  if (!may_split || tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
+  if (tiles * cfg.kv_heads * 4 >= kPrefillSlots * 3) return c;
   const int64_t padded = cfg.kv_heads % kXcds == 0 ? tiles : (tiles + kXcds - 1) / kXcds * kXcds;
   auto workgroups = [&] {  // with partitions of c.part keys; sets c.bytes
     int64_t items = 0, rows = 0;
@@ -362,24 +360,26 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     part = std::min<int64_t>(part, kMaxAutoPartition);
   }
   // The plain cut: these decode partitions, chunk rows over 384 keys. A step
-  // that it does not split needs no workspace and may be run without one, so
-  // the finer cuts below, which pay off on such steps too (32 decode rows of
-  // 1500 keys beside chunks, fp32 rows of 300-640 keys), are taken only where
-  // it splits something.
+  // that it does not split may be run without a workspace. The finer cuts
+  // below pay off on such steps too (us a call, whole and split: 17 fp32 decode
+  // rows of up to 640 keys, 28/4 heads x 128, 33.0 and 18.5; 4 decode rows of up
+  // to 2000 keys beside 3 x 17 chunk rows, 32/8 x 128, 33.9 and 22.1; an fp32
+  // prompt of 341 rows, 14/2 x 64, 27.7 and 19.6), so the plan splits them and
+  // says that without a workspace its rows and tiles may run whole.
   bool splits = false;
   for (int i = 0; i < n_slices; i++)
     splits |= (slices[i].start + slices[i].len - 1) / bs + 1 >
               round_to_blocks(slices[i].len > 1 ? kDefaultChunkPartition : static_cast<int>(part), bs);
-  const PrefillCut pre = cut_prefill(asked, slices, n_slices, n_tok, splits);
+  const PrefillCut pre = cut_prefill(asked, slices, n_slices, n_tok);
   if (auto_part) {
-    if (splits && chunk_rows && pre.on && pre.bytes <= kFinerPrefillScratch) {
+    if (chunk_rows && pre.on && pre.bytes <= kFinerPrefillScratch) {
       // Beside prefill tiles, whose workgroups share a CU with the decode
       // rows', 1024 keys: 2 x 512 rows after 1024 keys and 32 decode rows 25.6
       // against 31.1 us. Those partitions need at most 5 MB more of partials
       // than 2048-key ones: where the tiles' own leave that much of the static
       // scratch, else 2048 as before.
       part = std::min<int64_t>(std::max<int64_t>(shared, kMixedPrefillPartition), kMaxAutoPartition);
-    } else if (splits && !chunk_rows && cfg.kv_dtype == LE_F32) {
+    } else if (!chunk_rows && cfg.kv_dtype == LE_F32) {
       // fp32 keys are twice the bytes: a step that leaves CUs without a
       // workgroup takes shorter partitions, the shortest (two 32-key tiles a
       // wave on) that still gives every workgroup a CU of its own, where the
@@ -524,6 +524,7 @@ int le_plan_step(const le_step_slice* slices, int n_slices, const le_plan_config
     P.cfg.chunk_q_tile = pre.wide ? le::kWidePrefillTiles : le::kPrefillTiles;
     P.cfg.chunk_partition_tokens = 0;
   }
+  if (!fixed && !splits && parts > 0 && (pre.on || chk.empty())) P.cfg.chunk_partition_tokens = le::kMayRunWhole;
   P.n_tokens = static_cast<int32_t>(n_tok);
   P.n_seqs = n_seqs;
   P.n_table = static_cast<int32_t>(n_table);

@@ -9,7 +9,7 @@ import oracle
 from cases import make_case
 from gpu_util import emulated_bar, max_abs, oracle_out, poison_unused
 from llm_engine_amd._lib import LE_PLAN_XCD_LOCAL
-from test_gpu_attention import run_ragged, within
+from test_gpu_attention import TOL_F32, run_ragged, within
 
 pytestmark = pytest.mark.gpu
 
@@ -77,6 +77,78 @@ def test_prefill_ids_from_the_tables(gpu, kv, decode):
         return 2 * max_abs(old, want) + 2.0 ** -22 * float(np.nanmax(np.abs(want)))
 
     check(case, "f32", gpu, want_split=True, bar=bar)
+
+
+# Steps that the planner splits though they need no workspace: with a null or a
+# short workspace their rows and tiles run whole, like the undivided rows of the
+# 32-row plan; a step that needs one is refused as before.
+@pytest.mark.parametrize("heads,kv,ctx,q_len", [
+    ((32, 8, 128), "bf16", [1500, 2000, 84, 140, 30], [1, 1, 17, 40, 1]), ((14, 2, 64), "f16", [300, 1900, 9], [300, 1, 3]),
+    ((14, 2, 64), "f32", [341], [341]), ((16, 16, 64), "f32", [200, 1400, 300], [132, 1, 50]),
+    ((28, 4, 128), "f32", [640, 500, 257, 1], [1, 1, 1, 1]), ((14, 2, 64), "f32", [600], [1])])
+def test_steps_without_workspace_run_whole(gpu, heads, kv, ctx, q_len):
+    import ctypes
+    from llm_engine_amd import _lib, kernels
+    from gpu_util import device_q, slices_of, to_dev_cache
+    H, KH, hd = heads
+    case = make_case(ctx, H, KH, hd, 16, q_len=q_len, seed=len(ctx), kv_bf16=kv == "bf16", kv_f16=kv == "f16")
+    poison_unused(case)
+    q, qh = device_q(case, torch.float32, gpu)
+    kc, vc = to_dev_cache(case.k_cache, gpu), to_dev_cache(case.v_cache, gpu)
+    want = oracle_out(case, qh)
+    tol = TOL_F32 if kv == "f32" else emulated_bar(case, qh, want)
+
+    def run(plan, ws, nbytes):
+        out = torch.full_like(q, float("nan"))
+        st = _lib.load().le_ragged_paged_attention(
+            q.data_ptr(), _lib.LE_F32, kc.data_ptr(), vc.data_ptr(), plan.plan.cfg.kv_dtype, kc.numel() // (16 * KH * hd),
+            ctypes.byref(plan.plan), case.scale, out.data_ptr(), ws, nbytes, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        return st, out.cpu().numpy()
+
+    for flags in (0, LE_PLAN_XCD_LOCAL):
+        plan = kernels.Plan(slices_of(case), H, KH, hd, 16, kc.dtype, flags=flags).upload()
+        assert plan.workspace_size() > 0 and plan.plan.cfg.chunk_partition_tokens == -1
+        short = torch.zeros(4096, dtype=torch.uint8, device=gpu)
+        (st, whole), (st2, again) = run(plan, None, 0), run(plan, short.data_ptr(), 4096)
+        assert st == st2 == 0 and np.array_equal(whole, again) and not short.any()
+        assert np.isfinite(whole).all() and np.abs(whole - want).max() <= tol
+    split = kernels.Plan(slices_of(case), H, KH, hd, 16, kc.dtype, partition_tokens=16, chunk_q_tile=32).upload()
+    assert run(split, None, 0)[0] == _lib.LE_ENOSPACE or split.workspace_size() == 0
+
+
+@pytest.mark.parametrize("ctx", [[640, 500, 257, 1], [300]])
+def test_store_without_workspace(gpu, ctx):
+    """The store in the launch, rows run whole: the same bits as the store first and the attention after it, and the
+    same cache."""
+    import ctypes
+    from llm_engine_amd import _lib, kernels
+    from gpu_util import device_q, slices_of, to_dev_cache
+    H, KH, hd = 28, 4, 128
+    case = make_case(ctx, H, KH, hd, 16, seed=2)
+    q, qh = device_q(case, torch.float32, gpu)
+    plan = kernels.Plan(slices_of(case), H, KH, hd, 16, torch.float32).upload()
+    assert plan.workspace_size() > 0 and plan.plan.cfg.chunk_partition_tokens == -1
+    new = torch.randn(2, len(ctx), KH * hd, device=gpu, generator=torch.Generator(gpu).manual_seed(1))
+    outs, caches = [], []
+    for fused in (True, False):
+        kc, vc = to_dev_cache(case.k_cache, gpu).clone(), to_dev_cache(case.v_cache, gpu).clone()
+        out, nb = torch.full_like(q, float("nan")), kc.numel() // (16 * KH * hd)
+        tail = (kc.data_ptr(), vc.data_ptr(), _lib.LE_F32, nb, ctypes.byref(plan.plan), case.scale, out.data_ptr(), None, 0,
+                torch.cuda.current_stream().cuda_stream)
+        if fused:
+            st = _lib.load().le_ragged_paged_attention_store(q.data_ptr(), _lib.LE_F32, new[0].data_ptr(), new[1].data_ptr(),
+                                                             _lib.LE_F32, *tail)
+        else:
+            kernels.store_kv(new[0], new[1], plan.dev_array("slots"), kc, vc)
+            st = _lib.load().le_ragged_paged_attention(q.data_ptr(), _lib.LE_F32, *tail)
+        torch.cuda.synchronize()
+        assert st == 0
+        outs.append(out.cpu().numpy())
+        caches.append((kc.cpu().numpy(), vc.cpu().numpy()))
+    assert np.array_equal(*outs) and all(np.array_equal(a, b) for a, b in zip(*caches))
+    case.k_cache, case.v_cache = (c.reshape(d.shape) for c, d in zip(caches[0], (case.k_cache, case.v_cache)))
+    assert max_abs(outs[0], oracle_out(case, qh)) <= TOL_F32
 
 
 def test_prefill_wide_tiles(gpu):

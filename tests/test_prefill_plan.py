@@ -142,8 +142,6 @@ def test_fp32_decode_partitions_of_a_small_step():
 
         f32, b16 = make(torch.float32), make(torch.bfloat16)
         fits = [pt for pt in range(256, b16.cfg.partition_tokens, 128) if items(pt) * KH <= 256]
-        if b16.n_parts == 0:  # a step that runs without a workspace keeps doing so
-            fits = []
         assert f32.cfg.partition_tokens == (fits[0] if fits else b16.cfg.partition_tokens)
         assert f32.n_decode_items == items(f32.cfg.partition_tokens)
         seen.add(min(f32.cfg.partition_tokens, 640))
@@ -167,8 +165,9 @@ def plain_cut_splits(sl, H, KH, bs, partition=0):
 @pytest.mark.parametrize("heads", SHAPES)
 @pytest.mark.parametrize("kv", [torch.bfloat16, torch.float16, torch.float32])
 def test_steps_without_workspace(heads, kv):
-    """A step whose plain cut splits nothing runs without a workspace (a null one included), whatever finer partitions
-    its cut could take: decode rows beside short chunks, fp32 prompts, fp32 decode rows."""
+    """A step whose plain cut splits nothing needs no workspace, or its plan says that it may run whole without one,
+    whatever finer partitions its cut takes: decode rows beside short chunks, fp32 prompts, fp32 decode rows. No other
+    plan says so."""
     H, KH, hd = heads
     rng = np.random.default_rng(H + KH)
     seen = {True: 0, False: 0}
@@ -186,9 +185,23 @@ def test_steps_without_workspace(heads, kv):
         partition = int(rng.choice([0, 0, 640, 2048]))
         plan = kernels.Plan(sl, H, KH, hd, bs, kv, device="cpu", pin=False, partition_tokens=partition)
         splits = plain_cut_splits(sl, H, KH, bs, partition)
-        assert splits or plan.workspace_size() == 0, (trial, plan.plan.n_parts, [(s.start, s.len) for s in sl])
+        may_run_whole = plan.plan.cfg.chunk_partition_tokens == -1
+        assert may_run_whole == (not splits and plan.workspace_size() > 0), (trial, [(s.start, s.len) for s in sl])
         seen[splits] += 1
     assert min(seen.values()) > 15
+
+
+def test_plans_with_given_sizes_do_not_run_whole():
+    """Explicit chunk tiles or partitions, two launches and fixed layouts: refused without their workspace as ever."""
+    sl = [kernels.Slice(0, 0, 300, True, np.arange(19, dtype=np.int32), np.zeros(300, np.int32)),
+          kernels.Slice(1, 1499, 1, True, np.arange(94, dtype=np.int32), np.zeros(1500, np.int32))]
+    for kw in (dict(chunk_partition_tokens=128), dict(chunk_q_tile=32, partition_tokens=640),
+               dict(flags=LE_PLAN_TWO_LAUNCHES, partition_tokens=640), dict(partition_tokens=640)):
+        plan = kernels.Plan(sl, 14, 2, 64, 16, torch.bfloat16, device="cpu", pin=False, **kw)
+        assert plan.workspace_size() > 0 and plan.plan.cfg.chunk_partition_tokens != -1, kw
+    fixed = kernels.Plan(sl[1:], 14, 2, 64, 16, torch.float32, device="cpu", pin=False, partition_tokens=2048,
+                         table_capacity=128)
+    assert fixed.workspace_size() > 0 and fixed.plan.cfg.chunk_partition_tokens != -1
 
 
 @pytest.mark.parametrize("bs", [8, 16])
