@@ -211,9 +211,13 @@ template <bool kWhole> __device__ __forceinline__ ChunkItem tile_item(const Chun
   return it;
 }
 
-// The item's block ids: the plan's list, or, past its width, the sequence's table.
+// The item's block ids: the plan's list, or, past its width, the sequence's
+// table. Both lie in the plan's buffer: one base and a scalar offset (a choice
+// between two pointers took up to 11 more VGPRs in the mixed-step kernels).
 __device__ __forceinline__ const int32_t* tile_ids(const ChunkParams& p, const ChunkItem& it, int item) {
-  return it.seq < 0 ? p.tables + ~it.seq + it.blk_begin : p.item_ids + static_cast<int64_t>(item) * p.ids_stride;
+  const int64_t listed = p.item_ids - p.tables + static_cast<int64_t>(item) * p.ids_stride;
+  const int64_t off = it.seq < 0 ? static_cast<int64_t>(~it.seq) + it.blk_begin : listed;
+  return p.tables + __builtin_amdgcn_readfirstlane(static_cast<int>(off));
 }
 
 // One prefill workgroup: item `item`, kv head `kvh`, NC column tiles a wave.
