@@ -50,10 +50,28 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2)
   dec::decode_wg<ACT, KV, HD, kMfmaWaves, false, true>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
+// The reference-shaped launch's split rows in a 16-bit cache. Their partitions
+// are cut to the step's share of keys, longer than equal parts of every row, so
+// fewer of a row's heavy softmax weights are the largest of theirs (exactly 1):
+// with weights rounded to 16 bits the error against 64 bits grew from 2.50e-4
+// to 2.61e-4 (24 rows of 100-3000 keys, fp16, 32/8 heads x 128).
+template <typename ACT, typename KV, int HD>
+__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2))) void mfma_kernel_ref(DecodeParams p) {
+  __shared__ dec::DecodeSmem<KV, HD, kMfmaWaves> sm;
+  dec::decode_wg<ACT, KV, HD, kMfmaWaves, false, false, true>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
+}
+
 template <typename ACT, typename KV>
 hipError_t launch(const DecodeParams& p, hipStream_t s) {
   const dim3 grid(p.n_rows, p.kv_heads, p.items ? 1 : p.nsplit);
   const bool wide = p.wide != 0;
+  if constexpr (sizeof(KV) == 2) {
+    if (!p.items && p.nsplit > 1) {
+      if (p.head_dim == 64) mfma_kernel_ref<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);
+      else mfma_kernel_ref<ACT, KV, 128><<<grid, kMfmaThreads, 0, s>>>(p);
+      return hipGetLastError();
+    }
+  }
   if (p.items && !p.item_ids) {
     if (p.k_new) return hipErrorInvalidValue;  // a mixed step has stored its rows
     if (p.head_dim == 64) mfma_kernel_whole<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);

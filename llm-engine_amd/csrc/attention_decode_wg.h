@@ -578,7 +578,9 @@ __device__ __forceinline__ void load_tile(TileRegs<HD / 32>& r, const T* kc, con
   }
 }
 
-template <typename T, int HD>
+// kTwoTerm: each softmax weight in two 16-bit terms (hi + lo, the rest below
+// 2^-17 of it in bf16 and 2^-23 in fp16), two products a weight.
+template <typename T, int HD, bool kTwoTerm>
 __device__ __forceinline__ void compute_tile(WaveAcc<HD>& st, const TileRegs<HD / 32>& r,
                                              const typename mma16<T>::v8* qb, int key0, int key_end,
                                              float scale_log2, char* vt, int col, int grp) {
@@ -635,10 +637,15 @@ __device__ __forceinline__ void compute_tile(WaveAcc<HD>& st, const TileRegs<HD 
 #pragma unroll
   for (int kk = 0; kk < 2; kk++) {
     typename M::v8 pb;
+    [[maybe_unused]] typename M::v8 pl;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
       pb[j] = static_cast<typename M::scalar>(s[2 * kk][j]);
       pb[4 + j] = static_cast<typename M::scalar>(s[2 * kk + 1][j]);
+      if constexpr (kTwoTerm) {
+        pl[j] = static_cast<typename M::scalar>(s[2 * kk][j] - static_cast<float>(pb[j]));
+        pl[4 + j] = static_cast<typename M::scalar>(s[2 * kk + 1][j] - static_cast<float>(pb[4 + j]));
+      }
     }
     const char* r_lo = vt + (kk * 32 + grp * 4 + (col >> 2)) * V_STRIDE + (col & 3) * 8;
     const char* r_hi = r_lo + 16 * V_STRIDE;
@@ -647,6 +654,7 @@ __device__ __forceinline__ void compute_tile(WaveAcc<HD>& st, const TileRegs<HD 
       const typename M::v4 lo = lds_read_tr16<T>(r_lo + d * 32);
       const typename M::v4 hi = lds_read_tr16<T>(r_hi + d * 32);
       const typename M::v8 a = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (kTwoTerm) st.acc[d] = M::mma(a, pl, st.acc[d]);
       st.acc[d] = M::mma(a, pb, st.acc[d]);
     }
   }
@@ -691,9 +699,10 @@ template <typename T, int HD> struct DecodeTile16 {
                                               int kv_stride, int bs_shift, const int* tab, int tab_base, int col) {
     load_tile<T, HD>(r, kc, vc, key0, key_end, kv_stride, bs_shift, tab, tab_base, col);
   }
+  template <bool kTwoTerm>
   __device__ __forceinline__ static void compute(WaveAcc<HD>& st, const Regs& r, const QOp& q, int key0, int key_end,
                                                  float scale_log2, char* vt, int col, int grp) {
-    compute_tile<T, HD>(st, r, q.b, key0, key_end, scale_log2, vt, col, grp);
+    compute_tile<T, HD, kTwoTerm>(st, r, q.b, key0, key_end, scale_log2, vt, col, grp);
   }
   // The first tile, addressed without the item: key rel0 + 16i + col of the
   // item reads block ids[rel >> bs_shift] (the plan pads ids with -1 past
@@ -819,6 +828,7 @@ template <int HD> struct DecodeTile<float, HD> {
       r.v[j] = as_float4(ld16_stream(vrow + slot * kv_stride));
     }
   }
+  template <bool>  // (exact products: no terms to choose)
   __device__ __forceinline__ static void compute(WaveAcc<HD>& st, const Regs& r, const QOp& q, int key0, int key_end,
                                                  float scale_log2, char* vt, int col, int grp) {
     constexpr int DT = HD / 16;
@@ -895,7 +905,9 @@ template <typename KV, int HD, int NW> struct DecodeSmem {
 // kWhole: a plan's split rows run whole (no workspace); p.item_ids is null. An
 // instantiation of its own too: as a run-time choice it cost a small step 1 %
 // (two layers of 48 fp32 rows, 22.9 against 22.66 us).
-template <typename ACT, typename KV, int HD, int NW, bool kFold = false, bool kWhole = false>
+// kTwoTerm: softmax weights in two 16-bit terms (the reference-shaped launch,
+// whose partitions are cut by the step's lengths: attention_decode.hip).
+template <typename ACT, typename KV, int HD, int NW, bool kFold = false, bool kWhole = false, bool kTwoTerm = false>
 __device__ __forceinline__ void decode_wg(const DecodeParams& p, DecodeSmem<KV, HD, NW>& sm, int bx, int by, int bz) {
   using T = DecodeTile<KV, HD>;
   using L = MfmaLds<HD, T::VT_BYTES, NW>;
@@ -1056,28 +1068,28 @@ __device__ __forceinline__ void decode_wg(const DecodeParams& p, DecodeSmem<KV, 
         const int pairs = (n_tiles - 1) >> 1;
         for (int i = 0; i < pairs; i++) {
           T::load(rb, kc, vc, key0 + stride, key_end, kv_stride, bs_shift, tab, sb0, col);
-          T::compute(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
+          T::template compute<kTwoTerm>(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
           T::load(ra, kc, vc, key0 + 2 * stride, key_end, kv_stride, bs_shift, tab, sb0, col);
-          T::compute(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
+          T::template compute<kTwoTerm>(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
           key0 += 2 * stride;
         }
         T::load(rb, kc, vc, key0 + stride, key_end, kv_stride, bs_shift, tab, sb0, col);
-        T::compute(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
-        if (n_tiles - 2 * pairs == 2) T::compute(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
+        T::template compute<kTwoTerm>(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
+        if (n_tiles - 2 * pairs == 2) T::template compute<kTwoTerm>(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
       } else {  // fp32 tiles: the two-exit loop measured faster (config 2 20.0 against 20.5 us)
         while (true) {
           T::load(rb, kc, vc, key0 + stride, key_end, kv_stride, bs_shift, tab, sb0, col);
-          T::compute(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
+          T::template compute<kTwoTerm>(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
           if (key0 + stride >= key_end) break;
           T::load(ra, kc, vc, key0 + 2 * stride, key_end, kv_stride, bs_shift, tab, sb0, col);
-          T::compute(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
+          T::template compute<kTwoTerm>(st, rb, qb, key0 + stride, key_end, p.scale_log2, vt, col, grp);
           if (key0 + 2 * stride >= key_end) break;
           key0 += 2 * stride;
         }
       }
     } else {
       while (true) {
-        T::compute(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
+        T::template compute<kTwoTerm>(st, ra, qb, key0, key_end, p.scale_log2, vt, col, grp);
         key0 += stride;
         if (key0 >= key_end) break;
         T::load(ra, kc, vc, key0, key_end, kv_stride, bs_shift, tab, sb0, col);
