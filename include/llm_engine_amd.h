@@ -234,7 +234,10 @@ static inline const int32_t* le_plan_dev_array(const le_step_plan* plan, int64_t
  * GQA group. Prefill-chunk rows run the MFMA tile kernels (bf16 / fp16 tiles
  * for 16-bit caches, fp32 tiles for an fp32 cache), with a causal mask by
  * absolute position against the cached prefix. Split rows are merged inside
- * their launch. The result equals le_attention_decode on the same step.
+ * their launch. The result equals le_attention_decode on the same step, but for
+ * values that are not finite: the chunk kernels multiply a whole tile, so NaN or
+ * inf in a V row also reaches up to 127 rows before it in the same chunk (31
+ * with chunk_q_tile 16 or 32), never another sequence.
  * ------------------------------------------------------------------------ */
 /* Bytes of workspace that a packed step needs. They depend on how it is cut, and
  * a large step may need less than a small one (chunk rows that fill the chip are

@@ -1,4 +1,4 @@
-"""Greedy tokens of BASELINE config 1 from the CPU oracle (oracle.c, the fp32
+"""Greedy tokens of config 1 from the CPU oracle (oracle.c, the fp32
 reference forward), for the GPU end-to-end test:
 
   Qwen2.5-0.5B architecture, random-init fp32 weights (engine.synthetic_weights,

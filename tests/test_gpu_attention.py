@@ -5,13 +5,13 @@ Tolerances (|got - want| against the fp32 oracle, per element):
   * fp32 K/V: 4e-6 (decode rows: exact fp32 products; chunk rows: exact
     fp32 products at head_dim 128, three-term bf16 products at head_dim 64,
     each within a few fp32 roundings of the exact product; other summation
-    orders; the largest error seen is 1.3e-6; the north star allows 1e-3);
+    orders; the largest error seen is 1.3e-6; the target bar is 1e-3);
   * bf16 K/V: twice the error of the host emulation of the kernels'
     roundings on the same case (tests/precision.py: q and the softmax
     weights rounded to bf16 for the MFMA; gpu_util.emulated_bar). The
     emulation matches the GPU's error closely (config 2: 1.66e-3 emulated,
     1.65e-3 measured; config 3: 5.6e-3 and 5.5e-3), and every bar stays
-    inside the north star's 2e-2.
+    inside the target 2e-2.
 With bf16 activations the oracle is fed the same bf16-rounded q, and the
 output's own rounding adds 2^-8 |want| (round to nearest bf16: 2^-9
 relative, doubled for the error carried into it)."""
@@ -21,7 +21,7 @@ import torch
 
 from cases import loguniform_ctx, make_case, make_shared_prefix_case
 from gpu_util import device_q, emulated_bar, i32, max_abs, oracle_out, poison_unused, slices_of, to_dev_cache
-from llm_engine_amd._lib import LE_PLAN_TWO_LAUNCHES, LE_PLAN_XCD_LOCAL
+from llm_engine_amd._lib import LE_F32, LE_PLAN_TWO_LAUNCHES, LE_PLAN_XCD_LOCAL
 
 pytestmark = pytest.mark.gpu
 
@@ -56,6 +56,14 @@ def run_ragged(case, act, dev, **plan_kw):
     out = kernels.ragged_paged_attention(q, kc, vc, plan, case.scale)
     torch.cuda.synchronize()
     return out.float().cpu().numpy(), qh, plan
+
+
+def ran_on(plan, tile):
+    """Whether the step's chunk rows (if any) ran on 32-row tiles (tile 32), or
+    on the default's: prefill tiles, but for fp32 caches of head_dim 128."""
+    P = plan.plan
+    default32 = P.cfg.kv_dtype == LE_F32 and P.cfg.head_dim == 128
+    return P.n_chunk_items == 0 or (P.cfg.chunk_q_tile == 32) == (tile == 32 or default32)
 
 
 def tol_for(case, qh, want=None):
@@ -169,14 +177,16 @@ def test_decode_edges(gpu):
     assert max_abs(got[0, :64], v0) < 1e-6
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("kv_bf16", [False, True])
-def test_chunk_rows_small(gpu, kv_bf16):
+def test_chunk_rows_small(gpu, kv_bf16, tile):
     """Prefill chunks (causal inside the chunk, over a cached prefix) beside
     decode rows. bf16 K/V runs the MFMA chunk kernel, fp32 the decode kernel."""
     ctx = [40, 97, 160, 300, 64, 500]
     q_len = [1, 1, 64, 37, 64, 17]   # chunk at offsets 0, 263, 96, 483
     case = make_case(ctx, q_len=q_len, num_blocks=1024, seed=13, kv_bf16=kv_bf16)
-    got, qh, plan = run_ragged(case, torch.float32, gpu)
+    got, qh, plan = run_ragged(case, torch.float32, gpu, chunk_q_tile=tile)
+    assert ran_on(plan, tile)
     want = oracle_out(case, qh)
     err = max_abs(got, want)
     print(f"chunk rows kv_bf16={kv_bf16}: items dec={plan.plan.n_decode_items} "
@@ -187,10 +197,11 @@ def test_chunk_rows_small(gpu, kv_bf16):
     assert within(ref_shaped, want, tol_for(case, qh))
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("act,kv_bf16,flags", [(torch.float32, True, 0), (torch.bfloat16, True, 0),
                                                (torch.float32, False, 0), (torch.float32, True, LE_PLAN_XCD_LOCAL),
                                                (torch.float32, False, LE_PLAN_XCD_LOCAL)])
-def test_mixed_step_config3(gpu, act, kv_bf16, flags):
+def test_mixed_step_config3(gpu, act, kv_bf16, flags, tile):
     """Config 3: 32 decode rows (ctx U[256, 2048]) + 2 prefill chunks of 512
     at cached offsets 0 and 1024: 32 + 2 * 512 = 1056 ragged rows, with bf16
     K/V (16-bit MFMA chunk tiles) and fp32 K/V (three-term bf16 MFMA chunk
@@ -201,9 +212,10 @@ def test_mixed_step_config3(gpu, act, kv_bf16, flags):
     ctx = [512, 1536] + list(dec_ctx)
     q_len = [512, 512] + [1] * 32
     case = make_case(ctx, q_len=q_len, num_blocks=16384, seed=3, kv_bf16=kv_bf16)
-    got, qh, plan = run_ragged(case, act, gpu, flags=flags)
+    got, qh, plan = run_ragged(case, act, gpu, flags=flags, chunk_q_tile=tile)
     assert plan.plan.n_tokens == 1056
     assert plan.plan.n_chunk_items > 0 and plan.plan.xcd_local == (flags != 0)
+    assert ran_on(plan, tile)
     want = oracle_out(case, qh)
     err = max_abs(got, want)
     print(f"config3 act={act} kv_bf16={kv_bf16} flags={flags}: max|err|={err:.3e}")
@@ -313,16 +325,18 @@ def test_workspace_reused_across_plans(gpu):
     assert int(ws[:512 * 1024].count_nonzero().item()) == 0  # counters left at zero
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(32, 4, 64), (8, 8, 64), (16, 2, 128), (4, 1, 128)])
-def test_chunk_rows_other_shapes(gpu, q_heads, kv_heads, head_dim):
-    """The MFMA chunk kernel beyond the Qwen shape: GQA group 8 and 1,
+def test_chunk_rows_other_shapes(gpu, q_heads, kv_heads, head_dim, tile):
+    """The MFMA chunk kernels (prefill and 32-row tiles) beyond the Qwen shape: GQA group 8 and 1,
     head_dim 128, with partial row tiles, split tiles (merged in-kernel) and a
     cached prefix; bf16 K/V against the oracle."""
     ctx = [700, 333, 90, 1]
     q_len = [45, 333, 17, 1]  # chunk at offset 655, a whole-prompt chunk, a short tail, a decode row
     case = make_case(ctx, q_len=q_len, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim,
                      num_blocks=512, seed=41, kv_bf16=True)
-    got, qh, plan = run_ragged(case, torch.float32, gpu)
+    got, qh, plan = run_ragged(case, torch.float32, gpu, chunk_q_tile=tile)
+    assert ran_on(plan, tile)
     want = oracle_out(case, qh)
     err = max_abs(got, want)
     print(f"chunk {q_heads}/{kv_heads}x{head_dim}: items {plan.plan.n_chunk_items} parts {plan.plan.n_parts} "
@@ -331,19 +345,31 @@ def test_chunk_rows_other_shapes(gpu, q_heads, kv_heads, head_dim):
     assert within(got, want, tol_for(case, qh))
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("block_size", [8, 32, 64])
-def test_chunk_rows_block_sizes(gpu, block_size):
+def test_chunk_rows_block_sizes(gpu, block_size, tile):
     """Chunk rows and decode rows (one long enough to be split) in one step, so
     in one launch, at block sizes other than 16."""
     ctx = [600, 129, 64, 2000, 37]
     q_len = [100, 129, 3, 1, 1]
     case = make_case(ctx, q_len=q_len, block_size=block_size, num_blocks=512, seed=43, kv_bf16=True)
-    got, qh, plan = run_ragged(case, torch.bfloat16, gpu, partition_tokens=512)
+    got, qh, plan = run_ragged(case, torch.bfloat16, gpu, partition_tokens=512, chunk_q_tile=tile)
+    assert ran_on(plan, tile)
     want = oracle_out(case, qh)
     err = max_abs(got, want)
     print(f"chunk block {block_size}: items chunk {plan.plan.n_chunk_items} decode {plan.plan.n_decode_items} "
           f"max|err| {err:.3e}")
     assert plan.plan.n_chunk_items > 0 and plan.plan.n_decode_items > 2
+    assert within(got, want, tol_for(case, qh), torch.bfloat16)
+
+
+def test_more_rows_than_arrival_counters(gpu):
+    """A step with more (row, kv head) pairs than a workspace has arrival
+    counters (65536) runs on 32-row tiles, if no row is split."""
+    case = make_case([380] * 11, q_len=[380] * 11, q_heads=16, kv_heads=16, num_blocks=300, seed=71, kv_bf16=True)
+    got, qh, plan = run_ragged(case, torch.bfloat16, gpu)
+    assert plan.plan.n_tokens * 16 > 65536 and plan.plan.cfg.chunk_q_tile == 32 and plan.workspace_size() == 0
+    want = oracle_out(case, qh)
     assert within(got, want, tol_for(case, qh), torch.bfloat16)
 
 
@@ -412,8 +438,9 @@ def test_store_then_attend(gpu, kv_bf16, new_bf16, mixed, part):
     assert within(out.float().cpu().numpy(), oracle_out(case, qh), tol_for(case, qh))
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("seed", range(16))
-def test_random_ragged_steps(gpu, seed):
+def test_random_ragged_steps(gpu, seed, tile):
     """Randomised mixed steps against the oracle: the number of sequences,
     their contexts and rows (decode rows, chunks at cached offsets, whole
     prompts), the GQA shape, head dim, block size, cache and activation
@@ -440,7 +467,8 @@ def test_random_ragged_steps(gpu, seed):
     poison_unused(case)
     part = int(rng.choice([0, 256, 640, 2048]))
     flags = int(rng.choice([0, LE_PLAN_XCD_LOCAL]))
-    got, qh, plan = run_ragged(case, act, gpu, partition_tokens=part, flags=flags)
+    got, qh, plan = run_ragged(case, act, gpu, partition_tokens=part, flags=flags, chunk_q_tile=tile)
+    assert ran_on(plan, tile)
     want = oracle_out(case, qh)
     assert np.isfinite(got).all()
     err = max_abs(got, want)
@@ -514,8 +542,9 @@ def test_graph_replays_match_eager(gpu):
         assert torch.equal(again, eager)
 
 
+@pytest.mark.parametrize("tile", [0, 32])
 @pytest.mark.parametrize("kv", ["f32", "bf16", "f16"])
-def test_unused_cache_rows_never_read(gpu, kv):
+def test_unused_cache_rows_never_read(gpu, kv, tile):
     """Dead keys of a tile (past a partition's or row's end) are read at a
     live key's address and masked: with every unused cache row NaN, decode
     rows (both entry points, split rows included) and a mixed step with
@@ -526,7 +555,8 @@ def test_unused_cache_rows_never_read(gpu, kv):
     for ql in (None, q_len):
         case = make_case(ctx, q_len=ql, num_blocks=4096, seed=11, kv_bf16=kv == "bf16", kv_f16=kv == "f16")
         poison_unused(case)
-        b, qh, _ = run_ragged(case, torch.float32, gpu)
+        b, qh, plan = run_ragged(case, torch.float32, gpu, chunk_q_tile=tile)
+        assert ran_on(plan, tile)
         want = oracle_out(case, qh)
         assert np.isfinite(b).all()
         assert within(b, want, tol_for(case, qh))

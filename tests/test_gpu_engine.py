@@ -41,7 +41,7 @@ def run_both(w, prompts, max_tokens, num_blocks, cfg=None, prefix=False, frag=0,
 
 @pytest.mark.parametrize("attention,graph", [("ragged", False), ("reference", False), ("ragged", True)])
 def test_config1_matches_oracle_token_for_token(gpu, attention, graph):
-    """Qwen2.5-0.5B (24 layers) random-init fp32, 8 prompts of
+    """config 1: Qwen2.5-0.5B (24 layers) random-init fp32, 8 prompts of
     16..512 tokens, 32 greedy tokens, fragmented 4096-block pool. Through both
     attention entries: the ragged plan (le_ragged_paged_attention_qkv) and the
     reference-shaped launcher (le_attention_decode), which therefore give the

@@ -8,7 +8,7 @@ Tolerances (max-abs against the fp32 oracle): twice the error of the host
 emulation of the kernels' roundings on the same case (tests/precision.py: q
 and the softmax weights rounded to fp16 before the MFMA; emulated 2.3e-4 on
 config 2, where the GPU shows 2.9e-4, and 8.1e-4 on config 3, GPU 8.6e-4),
-inside the north star's 2e-2 for 16-bit K/V. fp16 outputs add their own
+inside the target 2e-2 for 16-bit K/V. fp16 outputs add their own
 rounding (<= 2^-11 relative, |out| < 4)."""
 import numpy as np
 import pytest

@@ -151,22 +151,106 @@ def test_store_without_workspace(gpu, ctx):
     assert max_abs(outs[0], oracle_out(case, qh)) <= TOL_F32
 
 
-def test_prefill_wide_tiles(gpu):
-    """256-column tiles: a step past 1000 keys per workgroup slot. The bar is
-    twice the error of the 32-row tiles, which make the same roundings."""
-    case = make_case([16100, 15000], 32, 4, 64, 16, q_len=[300, 45], seed=4, kv_bf16=True)
-
+def tile32_bar(case, gpu, act="f32", **kw):
+    """Twice the error of the 32-row tiles, which make the same roundings in another order."""
     def bar(qh, want):
-        old, _, plan = run_ragged(case, torch.float32, gpu, chunk_q_tile=32)
+        old, _, plan = run_ragged(case, ACT[act], gpu, chunk_q_tile=32, **kw)
         assert plan.plan.cfg.chunk_q_tile == 32
-        return 2 * max_abs(old, want)
+        err = np.abs(old.astype(np.float64) - want) - OUT_REL[act] * np.abs(want)
+        return 2 * max(0.0, float(err.max()))
+    return bar
 
-    check(case, "f32", gpu, want_wide=True, want_split=True, bar=bar)
+
+def test_prefill_wide_tiles(gpu):
+    """256-column tiles: a step past 1000 keys per workgroup slot."""
+    case = make_case([16100, 15000], 32, 4, 64, 16, q_len=[300, 45], seed=4, kv_bf16=True)
+    check(case, "f32", gpu, want_wide=True, want_split=True, bar=tile32_bar(case, gpu))
+
+
+# wide tiles beside decode rows and alone, of both 16-bit cache types, with
+# groups that fill the columns (8: 32 rows), leave some dead (7: 36 rows, 252
+# columns) and have one row a column (1: 256 rows); split over partitions
+# (few rows after many keys) and whole (three workgroups for every four slots)
+@pytest.mark.parametrize("heads,kv,act,bs,ctx,q_len,decode", [
+    ((32, 4, 64), "bf16", "bf16", 16, [16100, 15000], [300, 45], True), ((32, 4, 64), "f16", "f16", 16, [16100, 15000], [300, 45], True),
+    ((32, 4, 64), "f16", "f32", 64, [16100, 15000], [300, 45], False),
+    ((14, 2, 64), "bf16", "f32", 8, [17300, 9000], [560, 75], True), ((14, 2, 64), "f16", "bf16", 32, [17300, 9000], [560, 75], True),
+    ((8, 8, 64), "bf16", "f32", 16, [15990, 12800], [1000, 300], True), ((8, 8, 64), "f16", "f32", 64, [15990, 12800], [1000, 300], True),
+    ((8, 8, 64), "bf16", "bf16", 16, [15990, 12800], [1000, 300], False)])
+def test_prefill_wide_split(gpu, heads, kv, act, bs, ctx, q_len, decode):
+    H, KH, hd = heads
+    ctx, q_len = ctx + [1200, 90] * decode, q_len + [1, 1] * decode
+    case = make_case(ctx, H, KH, hd, bs, q_len=q_len, seed=H + bs, kv_bf16=kv == "bf16", kv_f16=kv == "f16")
+    poison_unused(case)
+    check(case, act, gpu, want_wide=True, want_split=True, bar=tile32_bar(case, gpu, act))
+
+
+@pytest.mark.parametrize("kv,act,decode", [("bf16", "bf16", False), ("bf16", "f32", True), ("f16", "f16", True)])
+def test_prefill_wide_whole(gpu, kv, act, decode):
+    """Wide tiles that hold all keys of their rows: 54 tiles x 8 kv heads."""
+    ctx, q_len = [3000, 2500] + [700, 3] * decode, [900, 800] + [1, 1] * decode
+    case = make_case(ctx, 64, 8, 64, 16, q_len=q_len, seed=9, kv_bf16=kv == "bf16", kv_f16=kv == "f16")
+    poison_unused(case)
+    check(case, act, gpu, want_wide=True, want_split=False, bar=tile32_bar(case, gpu, act))
+
+
+# Infinities and NaN: a key that scores -inf drops out, a row all of whose keys
+# do is NaN; NaN or inf in a key, a value or a query row reaches the rows that
+# attend to it. It reaches no other sequence, and of the chunk's earlier rows
+# only, from a value (as 0 * NaN), those whose wave computes its 64-key tile: the
+# rows of a wave (64 at most) and 63 before it. The 32-row tiles spread it over
+# their 32 rows.
+@pytest.mark.parametrize("kind", ["drop", "all", "nan_v", "inf_v", "inf_k", "nan_k", "nan_q"])
+@pytest.mark.parametrize("heads,kv,wide", [((8, 2, 64), "bf16", False), ((8, 2, 64), "f16", False), ((3, 3, 64), "bf16", False),
+                                           ((8, 2, 128), "bf16", False), ((14, 2, 64), "f32", False),
+                                           ((3, 3, 64), "f32", False), ((32, 4, 64), "bf16", True)])
+def test_prefill_nonfinite(gpu, heads, kv, wide, kind):
+    H, KH, hd = heads
+    ctx, q_len = [300, 150, 200, 40], [280, 60, 1, 40]
+    if wide:
+        ctx, q_len = ctx + [16300, 15000], q_len + [300, 45]
+    case = make_case(ctx, H, KH, hd, 16, q_len=q_len, seed=11)
+    at = {"nan_v": 191, "inf_v": 119}.get(kind, 150)  # a key of sequence 0's chunk
+    slot = [case.blocks_of(s)[np.arange(ctx[s]) // 16].astype(np.int64) * 16 + np.arange(ctx[s]) % 16 for s in range(len(ctx))]
+    k, v = case.k_cache.reshape(-1, KH, hd), case.v_cache.reshape(-1, KH, hd)
+    q = case.q.reshape(-1, H, hd)
+    if kind in ("drop", "all", "inf_k"):
+        q[..., 0] = np.abs(q[..., 0]) + 1
+    if kind in ("drop", "all"):
+        k[slot[0][[3, 70, 150]] if kind == "drop" else slot[0][:40], :, 0] = -np.inf
+    elif kind == "nan_v":
+        v[slot[0][at], 0, 5] = np.nan
+    elif kind == "inf_v":
+        v[slot[0][at], 0, 5] = np.inf
+    elif kind == "inf_k":
+        k[slot[0][at], 0, 0] = np.inf
+    elif kind == "nan_k":
+        k[slot[0][at], 0, 0] = np.nan
+    else:
+        q[77, 1, 3] = np.nan
+    if kv != "f32":
+        case.k_cache, case.v_cache = ((oracle.f32_to_bf16(c) if kv == "bf16" else oracle.f32_to_f16(c)) for c in (case.k_cache, case.v_cache))
+    new, _, plan = run_ragged(case, torch.float32, gpu)
+    old = run_ragged(case, torch.float32, gpu, chunk_q_tile=32)[0]
+    assert plan.plan.cfg.chunk_q_tile == (-1 if wide else 0)
+    n, o = np.isfinite(new), np.isfinite(old)
+    print(kind, "not finite: prefill", int((~n).sum()), "32-row", int((~o).sum()))
+    far = (case.token_seq != 0) | (case.token_pos < at - 63 - (64 if wide else 32) // (H // KH))
+    assert not (o & ~n)[far if kind in ("nan_v", "inf_v") else slice(None)].any()
+    pos = case.token_pos
+    seq0 = case.token_seq == 0
+    must = {"drop": seq0 & (pos < 0), "all": seq0 & (pos < 40), "nan_q": np.arange(len(pos)) == 77}.get(kind, seq0 & (pos >= at))
+    heads0 = n.reshape(len(pos), H, hd)[:, 1 if kind == "nan_q" else 0]
+    if kv != "f32" or kind not in ("drop", "all"):  # (an infinity's terms: inf - inf)
+        assert not heads0[must, 5].any() and n.reshape(len(pos), H, hd)[~seq0].all()
+        assert kind != "drop" or n.all()
+    both = n & o
+    assert np.abs(new[both] - old[both]).max() <= (4e-6 if kv == "f32" else 0.03)
 
 
 @pytest.mark.parametrize("kind", ["large", "negative", "rising"])
-@pytest.mark.parametrize("hd", [64, 128])
-def test_prefill_softmax_base(gpu, kind, hd):
+@pytest.mark.parametrize("hd,kv", [(64, "bf16"), (128, "bf16"), (64, "f16"), (128, "f16"), (64, "f32")])
+def test_prefill_softmax_base(gpu, kind, hd, kv):
     """Scores far from 0 (the base that they are taken relative to starts at
     0): tens of log2 units wide, all far below 0, and rising along the keys so
     that the base moves tile after tile."""
@@ -182,7 +266,12 @@ def test_prefill_softmax_base(gpu, kind, hd):
     else:
         q[..., 0] = 8.0
         k[..., 0] = (-12.0 if kind == "negative" else pos[:, None] / 16)
-    case.k_cache, case.v_cache = (oracle.f32_to_bf16(c) for c in (case.k_cache, case.v_cache))
+    if kv == "f32":  # every product to fp32 rounding: the 32-row tiles' bar, and an ulp of the largest value
+        bar = tile32_bar(case, gpu)
+        check(case, "f32", gpu, bar=lambda qh, want: bar(qh, want) + 2.0 ** -22 * float(np.abs(case.v_cache).max()))
+        return
+    narrow = oracle.f32_to_bf16 if kv == "bf16" else oracle.f32_to_f16
+    case.k_cache, case.v_cache = (narrow(c) for c in (case.k_cache, case.v_cache))
     check(case, "f32", gpu)
 
 

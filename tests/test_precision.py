@@ -4,7 +4,7 @@ q * scale * log2(e), and the softmax weights rounded to the cache type before
 the MFMA) on configs 2 and 3, against the
 fp32 oracle. The GPU parity tests hold each 16-bit case to twice its own
 emulated error (gpu_util.emulated_bar); here the emulated errors of the
-benchmark configs are stated and kept under half the north star's 2e-2, so
+benchmark configs are stated and kept under half the target 2e-2, so
 those bars stay inside it."""
 import numpy as np
 import pytest
@@ -13,7 +13,7 @@ from cases import loguniform_ctx, make_case
 from gpu_util import oracle_out
 from precision import emulate
 
-NORTH_STAR = 2e-2  # max-abs bound for 16-bit K/V
+TARGET = 2e-2  # max-abs bound for 16-bit K/V
 # the emulated max-abs error, decode rows and prefill-chunk rows, within 20 %
 STATED = {"config2": {"bf16": 1.66e-3, "f16": 2.29e-4},
           "config3": {"bf16": (1.12e-3, 5.79e-3), "f16": (1.27e-4, 8.74e-4)}}
@@ -26,7 +26,7 @@ def test_config2_emulated_error_under_half_the_bar(dt):
                      kv_f16=dt == "f16")
     err = float(np.abs(emulate(case, case.q, dt) - oracle_out(case, case.q)).max())
     print(f"config2 {dt}: emulated max|err| {err:.3e}")
-    assert 2 * err < NORTH_STAR
+    assert 2 * err < TARGET
     assert abs(err / STATED["config2"][dt] - 1) < 0.2
 
 
@@ -38,7 +38,7 @@ def test_config3_emulated_error_under_half_the_bar(dt):
     chunk = np.array([case.seq_qlen[s] > 1 for s in case.token_seq])
     e = np.abs(emulate(case, case.q, dt, chunk) - oracle_out(case, case.q))
     print(f"config3 {dt}: emulated max|err| decode rows {e[~chunk].max():.3e}, chunk rows {e[chunk].max():.3e}")
-    assert 2 * e.max() < NORTH_STAR
+    assert 2 * e.max() < TARGET
     d, c = STATED["config3"][dt]
     assert abs(e[~chunk].max() / d - 1) < 0.2 and abs(e[chunk].max() / c - 1) < 0.2
 
