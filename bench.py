@@ -367,13 +367,18 @@ def attention_leg(workload, kv, L, steps, warmup, partition=0, chunk_partition=0
     attn_us = a0.elapsed_time(a1) * 1e3 / (reps * L)
     achieved = attn_b / (attn_us * 1e-6) / 1e9
     P = plan.plan
+    if not P.n_chunk_items:
+        kernel = "decode mfma_kernel"
+    elif P.cfg.chunk_q_tile > 0:  # 32-row tiles
+        kernel = "ragged_kernel" if P.n_decode_items else "chunk_kernel"
+    else:
+        kernel = ("ragged_" if P.n_decode_items else "") + ("prefill_f32_kernel" if kv == "f32" else "prefill_kernel")
+    if P.n_chunk_items and P.n_decode_items:
+        kernel += ": chunk and decode workgroups in one launch"
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
                 "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
                 "traffic": measured_traffic(workload, kv) if partition == 0 and chunk_partition == 0 else None,
-                "kernel": "le_ragged_paged_attention ("
-                          + ("ragged_kernel: chunk and decode workgroups in one launch"
-                             if P.n_chunk_items and P.n_decode_items else
-                             "chunk_kernel" if P.n_chunk_items else "decode mfma_kernel") + ")",
+                "kernel": f"le_ragged_paged_attention ({kernel})",
                 "bytes_per_launch": attn_b, "us_per_launch": round(attn_us, 3)}
     if workload == "config3":
         fl = chunk_flops(ctx, q_len)
@@ -668,7 +673,7 @@ def main():
               "sequence with no exchange; multi-GPU runs are not part of it).", file=sys.stderr)
         sys.exit(2)
 
-    # The north star's target point and the mixed step are measured the same
+    # The target point and the mixed step are measured the same
     # way (fewer steps), each with its own roofline, after the main workload.
     extras = []
     if args.workload == "config2" and not args.no_extra_workloads:

@@ -57,8 +57,10 @@ __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32S
   constexpr int U = kTileKeys / 32;
 
   char* lds = sm.lds;
+  [[maybe_unused]] const uint64_t t_start = LE_TIM_NOW();
   const ChunkItem it = tile_item<kWhole>(p, item);
   if (it.n_q <= 0) return;
+  stamp_item(it, t_start);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
@@ -266,6 +268,7 @@ __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32S
     const int rel = t * kTileKeys;
     stash();
     __syncthreads();
+    if (t == 0) LE_TIM(1, LE_TIM_NOW());
     if (t + 1 < n_tiles) {
       issue(rel + kTileKeys);
       fetch_ids(rel + 2 * kTileKeys);
@@ -273,6 +276,8 @@ __device__ __forceinline__ void prefill_f32_wg(const ChunkParams& p, PrefillF32S
     if (rel <= wave_lim) tile(rel);
     if (t + 1 < n_tiles) __syncthreads();  // the tile is no longer read
   }
+  LE_TIM(2, LE_TIM_NOW());
+  LE_TIM_WAVE(8, LE_TIM_NOW());
   finish_tile<ACT, float, HD, 1>(p, it, kvh, sm.last, acc, base, lsum, row_of, head_of);
 }
 

@@ -137,6 +137,11 @@ __device__ __forceinline__ void finish_tile(const ChunkParams& p, const ChunkIte
           if (row_of[nc] >= 0) elem<ACT>::store8(out + d * 32 + e * 2, f);
         }
     }
+#ifdef LE_TIMING
+    __builtin_amdgcn_s_waitcnt(0);
+    LE_TIM(3, LE_TIM_NOW());
+    LE_TIM(4, LE_TIM_NOW());
+#endif
     return;
   }
 
@@ -185,16 +190,32 @@ __device__ __forceinline__ void finish_tile(const ChunkParams& p, const ChunkIte
   }
   __builtin_amdgcn_s_waitcnt(0);  // this thread's partial stores are performed
   __syncthreads();                // ... and every other thread's
+  LE_TIM(3, LE_TIM_NOW());
   arrival_t* counter = p.parts.counters + static_cast<int64_t>(it.tok_begin) * p.kv_heads + kvh;
   if (tid == 0) {
     const arrival_t seen = __hip_atomic_fetch_add(counter, arrival_t{1}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     last = seen == static_cast<arrival_t>(it.part_stride - 1);
   }
   __syncthreads();
+#ifdef LE_TIMING
+  if (!last) LE_TIM(4, LE_TIM_NOW());
+#endif
   if (!last) return;
   chk::merge_tile<ACT, HD, 4, chk::kHalfPartials<KV>, kThreads, HD == 64 && NC == 1 ? 2 : 4>(p, it, acc_rsrc, ml, rec_tile, it.part0 - it.part,
                                                                it.part_stride, G, kvh, it.n_q, it.tok_begin);
   if (tid == 0) __hip_atomic_store(counter, arrival_t{0}, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#ifdef LE_TIMING
+  __builtin_amdgcn_s_waitcnt(0);  // the merge's output stores are performed
+  LE_TIM(4, LE_TIM_NOW());
+#endif
+}
+
+// What a prefill workgroup stamps at its start (measurement builds).
+__device__ __forceinline__ void stamp_item(const ChunkItem& it, uint64_t t_start) {
+  LE_TIM(0, t_start);
+  LE_TIM(5, LE_TIM_PLACE());
+  LE_TIM(6, (static_cast<uint64_t>(it.blk_end - it.blk_begin) << 32) | static_cast<uint32_t>(it.part0 < 0 ? 0 : it.part_stride));
+  LE_TIM(7, 2);
 }
 
 // The workgroup's item; n_q 0: nothing to do (padding that keeps split tiles
@@ -239,8 +260,10 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
 
   char* lds = sm.lds;
   int& last = sm.last;
+  [[maybe_unused]] const uint64_t t_start = LE_TIM_NOW();
   const ChunkItem it = tile_item<kWhole>(p, item);
   if (it.n_q <= 0) return;
+  stamp_item(it, t_start);
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1), wave = tid >> 6;
   const int col = lane & 31, half = lane >> 5;
@@ -474,6 +497,7 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
   }
   stash(sa, 0);
   __syncthreads();
+  LE_TIM(1, LE_TIM_NOW());
   if constexpr (kAhead == 2) {
     for (int t = 0; t < n_tiles; t += 2) {
       step(t, sa, sb);
@@ -483,6 +507,8 @@ __device__ __forceinline__ void prefill_wg(const ChunkParams& p, PrefillSmem<HD>
     for (int t = 0; t < n_tiles; t++) step(t, sa, sa);
   }
 
+  LE_TIM(2, LE_TIM_NOW());
+  LE_TIM_WAVE(8, LE_TIM_NOW());
   finish_tile<ACT, KV, HD, NC>(p, it, kvh, last, acc, base, lsum, row_of, head_of);
 }
 
