@@ -3,7 +3,6 @@
 // this file.
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <mutex>
@@ -153,8 +152,7 @@ int le_attention_decode(const void* q, le_dtype act_dtype, const void* k_cache,
                            kv_heads, head_dim);
   p.items = nullptr;
   p.n_rows = n_tokens;
-  p.share_items = std::max(1, le::unplanned_items(n_tokens * kv_heads) / kv_heads);
-  p.min_part = le::unplanned_part(n_tokens * kv_heads);
+  p.min_part = le::unplanned_part(n_tokens * kv_heads, head_dim, kv_dtype);
   p.q_heads = q_heads; p.kv_heads = kv_heads; p.head_dim = head_dim; p.block_size = block_size;
   p.scale_log2 = scale * 1.4426950408889634f;
   p.num_cache_blocks = num_cache_blocks;

@@ -50,11 +50,12 @@ __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2)
   dec::decode_wg<ACT, KV, HD, kMfmaWaves, false, true>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// The reference-shaped launch's split rows in a 16-bit cache. Their partitions
-// are cut to the step's share of keys, longer than equal parts of every row, so
-// fewer of a row's heavy softmax weights are the largest of theirs (exactly 1):
-// with weights rounded to 16 bits the error against 64 bits grew from 2.50e-4
-// to 2.61e-4 (24 rows of 100-3000 keys, fp16, 32/8 heads x 128).
+// The reference-shaped launch's split rows in a 16-bit cache, with softmax
+// weights in two terms. Longer partitions than nsplit parts of every row leave
+// fewer of a row's heavy weights the largest of theirs (exactly 1): with weights
+// rounded to 16 bits the error against 64 bits grew from 2.50e-4 to 2.61e-4 (24
+// rows of 100-3000 keys, fp16, 32/8 heads x 128); here it is 2.1e-4, for 1 % of
+// the time.
 template <typename ACT, typename KV, int HD>
 __global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2))) void mfma_kernel_ref(DecodeParams p) {
   __shared__ dec::DecodeSmem<KV, HD, kMfmaWaves> sm;

@@ -58,20 +58,21 @@ struct Work {
 // This workgroup's item; valid is false if it has nothing to do (a split past
 // the end of a short context in the reference-shaped launch). Returned by
 // value so it stays in registers.
-// Without a plan the host does not know the lengths: each workgroup sums the
-// step's contexts itself (positions it loads in the round trip that fetches
-// its own) and cuts its row into partitions of one workgroup's share of them
-// (share_items workgroups per kv head), at least min_part keys, and at most
-// nsplit of them; the grid's workgroups past a row's last partition leave. All rows
-// are thereby cut to about one length, so a short row does not pay the
-// partial store and merge of many tiny ones, and the launch runs in fewer
-// rounds. Against nsplit equal partitions of every row (us): 24 rows of 100-3000
-// keys, fp16, 32/8 heads x 128, 46.7 -> 39.7 (3.3 TB/s); 64 rows of 4096, bf16,
-// 14/2 x 64, 38.0 -> 30.1; 64 of 64-4096 27.9 -> 20.5; 4 of 300-3000, 16/16,
-// 27.0 -> 16.7; one row 13.4 and 13.4. scratch: NW ints of LDS, which the
-// caller writes again only behind a barrier.
-template <int NW, bool kWhole>
-__device__ __forceinline__ Work resolve(const DecodeParams& p, int bx, int bz, int* scratch) {
+// Without a plan the host does not know the lengths: each row is cut into
+// nsplit equal partitions, or fewer of at least min_part keys (unplanned_part in
+// le_internal.h), and the grid's workgroups past a row's last partition leave. So
+// a short row does not pay the partial store and merge of many tiny partitions,
+// and a row's cut depends on its own length alone. Against nsplit partitions of
+// every row (us a call): 24 rows of 100-3000 keys, fp16, 32/8 heads x 128, 52.4 ->
+// 45.7 (3.0 TB/s); 64 rows of 4096, bf16, 14/2 x 64, 42.8 -> 33.9; 64 of 64-4096
+// 28.8 -> 20.7; 4 of 300-3000, 16/16, 25.9 -> 12.2; 37 calls of 1 to 255 rows 1.23x
+// in the geometric mean, from 0.98 (steps whose partitions were long already: the
+// weights' second term) to 2.5. Cutting every row to the step's share of keys
+// instead, summed from the positions by each workgroup, took 1.21x and lost
+// where few long partitions remained: 49 rows of 731-5854, 16/16 x 64, 273 -> 302
+// (274 here); 19 of 316-2531, fp32, 8/8 x 128, 148 -> 176 (146 here).
+template <bool kWhole>
+__device__ __forceinline__ Work resolve(const DecodeParams& p, int bx, int bz) {
   if (p.items) {
     const DecodeItem it = p.items[bx];
     if constexpr (kWhole)  // the row's first item takes all of it
@@ -81,25 +82,10 @@ __device__ __forceinline__ Work resolve(const DecodeParams& p, int bx, int bz, i
                 it.part, it.part_begin, it.n_parts, it.n_parts > 0};  // n_parts 0: padding
   }
   const int token = bx;
-  const int bs_shift = __builtin_ctz(p.block_size);  // block sizes are powers of two
   const int pos = p.token_pos[token];
   const int nb = pos / p.block_size + 1;
-  int ns = 1;
-  // (a row that one smallest partition holds needs no sum)
-  if (p.nsplit > 1 && pos >= p.min_part) {
-    int sum = 0;
-    for (int i = threadIdx.x; i < p.n_rows; i += NW * kWave) sum += p.token_pos[i] >> bs_shift;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, kWave);
-    if ((threadIdx.x & (kWave - 1)) == 0) scratch[threadIdx.x / kWave] = sum;
-    __syncthreads();
-    sum = 0;
-#pragma unroll
-    for (int w = 0; w < NW; w++) sum += scratch[w];
-    const int share = (sum + p.n_rows + p.share_items - 1) / p.share_items;
-    const int len = max(share, ((p.min_part - 1) >> bs_shift) + 1);
-    ns = min(min(p.nsplit, nb), (nb - 1) / len + 1);
-  }
+  const int len = ((p.min_part - 1) >> __builtin_ctz(p.block_size)) + 1;  // blocks of a smallest partition
+  const int ns = min(min(p.nsplit, nb), (nb - 1) / len + 1);
   const int split = bz;
   const int b0 = static_cast<int>(static_cast<int64_t>(split) * nb / ns);
   const int b1 = static_cast<int>(static_cast<int64_t>(split + 1) * nb / ns);
@@ -905,8 +891,8 @@ template <typename KV, int HD, int NW> struct DecodeSmem {
 // kWhole: a plan's split rows run whole (no workspace); p.item_ids is null. An
 // instantiation of its own too: as a run-time choice it cost a small step 1 %
 // (two layers of 48 fp32 rows, 22.9 against 22.66 us).
-// kTwoTerm: softmax weights in two 16-bit terms (the reference-shaped launch,
-// whose partitions are cut by the step's lengths: attention_decode.hip).
+// kTwoTerm: softmax weights in two 16-bit terms (the reference-shaped launch's
+// split rows: attention_decode.hip).
 template <typename ACT, typename KV, int HD, int NW, bool kFold = false, bool kWhole = false, bool kTwoTerm = false>
 __device__ __forceinline__ void decode_wg(const DecodeParams& p, DecodeSmem<KV, HD, NW>& sm, int bx, int by, int bz) {
   using T = DecodeTile<KV, HD>;
@@ -950,7 +936,7 @@ __device__ __forceinline__ void decode_wg(const DecodeParams& p, DecodeSmem<KV, 
   __builtin_amdgcn_s_waitcnt(0);
   LE_TIM(9, LE_TIM_NOW());
 #endif
-  const Work w = resolve<NW, kWhole>(p, bx, bz, tab);
+  const Work w = resolve<kWhole>(p, bx, bz);
   if (!w.valid) return;
   LE_TIM(0, t_start);
   LE_TIM(5, LE_TIM_PLACE());

@@ -104,7 +104,7 @@ struct DecodeParams {
   int ids_stride;
   int n_rows;               // items, or tokens when items is null
   int nsplit;
-  int share_items, min_part;  // items null: workgroups per kv head that share the keys, least keys of a partition
+  int min_part;             // items null: least keys of a partition
   int q_heads, kv_heads, head_dim, block_size;
   float scale_log2;         // softmax scale * log2(e)
   int64_t num_cache_blocks;
@@ -175,18 +175,23 @@ hipError_t attention_ragged(const DecodeParams& d, const ChunkParams& c, int act
 // know the context lengths: enough workgroups to cover the chip several times.
 int decode_nsplit(int n_tokens, int kv_heads);
 
-// How its rows are then cut on the device (resolve() in attention_decode_wg.h):
-// the step's keys shared by about this many workgroups, in partitions of at
-// least this many keys; rows = tokens x kv heads. Measured (us a call):
-// * 1024 workgroups against 512 below 512 rows: 33 rows of 3626 keys, fp32, 28/4
-//   heads x 128, 139 against 159 (four partitions a row just pass one round at
-//   two workgroups a CU); 40 of 663-5304, bf16, 8/8 x 128, 102 against 108; 24 of
-//   100-3000, fp16, 32/8 x 128, 39.7 against 39.8. From 512 rows on 512: 256 rows of
-//   64-2048, 14/2 x 64, 34.9 against 41.1.
-// * 512 keys against 256 from 128 rows on: 64 of 64-4096, 14/2 x 64, 20.5 against
-//   25.7. Below that, where CUs are idle, 256: 7 of 1-1674, bf16, 32/8 x 128, 10.9
-//   against 14.2; 48 of 32-2048, fp32, 14/2 x 64, 16.5 against 22.5.
-constexpr int unplanned_items(int64_t rows) { return rows < 512 ? 1024 : 512; }
-constexpr int unplanned_part(int64_t rows) { return rows < 128 ? 256 : 512; }
+// The least keys of a partition there (resolve() in attention_decode_wg.h); rows =
+// tokens x kv heads. A partition has to stream for longer than its finish takes
+// (partial, arrival, merge), but a chip with idle CUs gains from short ones, and
+// one that the rows fill by themselves from whole rows. Measured (us a call):
+// * below 128 rows 256 keys against 512: 7 rows of 1-1674, bf16, 32/8 heads x 128,
+//   10.9 and 14.2; 48 of 32-2048, fp32, 14/2 x 64, 16.5 and 22.5 (128 keys 24.2
+//   against 22.5 with two layers).
+// * from 128 rows on 512 against 256: 24 of 100-3000, fp16, 32/8 x 128, 46.0 and
+//   53.1; 116 of 348, fp32, 14/2 x 64, 26.7 and 31.0.
+// * from 512 rows on 1024 against 512: 256 of 64-2048, fp16, 14/2 x 64, 41.2 and
+//   44.7; 63 of 200-2000, bf16, 16/16 x 64, 63.2 and 69.1.
+// * half of that for fp32 keys of head_dim 128 (1 KB each): 256 against 512 for 19
+//   rows of 316-2531, 8/8 heads, 146 and 176; below 128 rows 256 stay (8 rows of
+//   3736, 28/4 heads, 80.3 against 88.7 with 128).
+constexpr int unplanned_part(int64_t rows, int head_dim, int kv_dtype) {
+  const int keys = rows < 128 ? 256 : rows < 512 ? 512 : 1024;
+  return rows >= 128 && kv_dtype == 0 /* LE_F32 */ && head_dim == 128 ? keys / 2 : keys;
+}
 
 }  // namespace le
