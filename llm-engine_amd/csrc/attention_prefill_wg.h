@@ -9,13 +9,16 @@
 // by idle waves (one wave per query head of the group: half of them with
 // G = 4, seven of eight with G = 1), by a load phase that nothing overlaps,
 // and by the partials of its 384-key partitions. Measured, chunk tile against
-// this one (us; the prefill kernel alone): 4096 rows after 0-1536 keys, 32/4
+// this one (us; the kernel alone, back to back, untraced: a profiler's launches
+// run up to 10 % longer): 4096 rows after 0-1536 keys, 32/4
 // heads x 64, 131 against 63 (706 TFLOP/s); 2048 rows after 8192, 32/8 x 128,
 // 845 against 357 (865); 4096 rows after 4096, 32/4 x 64, 369 against 164
 // (890); 512 rows after 1024, 14/2 x 64, 18.5 against 15.4; 4 x 512 rows after
 // 4096, 8/8 x 128, 419 against 69. What bounds it now: with the chip full, the
-// matrix cores' issue beside the softmax's vector work on the same SIMDs (a
-// large bf16 GEMM reaches 1200-1370 TFLOP/s on this card); in small steps the
+// matrix cores' issue beside the softmax's vector work on the same SIMDs
+// (counters of the 2048 rows after 8192: MFMA busy 36 % of a SIMD's cycles,
+// vector instructions active 45 %, LDS 36 %; a large bf16 GEMM reaches 1200-1370
+// TFLOP/s on this card); in small steps the
 // serial chain of a tile (fragments, product, max, exp2, product, barrier:
 // about 1 us per 64 keys with one workgroup on a CU).
 //

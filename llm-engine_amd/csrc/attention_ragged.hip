@@ -13,8 +13,9 @@
 // Both kinds keep their own merges inside the launch: partition indices and
 // arrival counters are disjoint between them (the plan numbers partitions
 // across both lists; counters are indexed by a row's or tile's first token).
-// Workgroups are 512 threads (the chunk workgroup's eight waves); the decode
-// workgroups run as eight waves as well. The LDS is the larger of the two.
+// Beside 32-row tiles (ragged_kernel) workgroups are 512 threads (the chunk
+// workgroup's eight waves) and the decode workgroups run as eight waves as well;
+// beside prefill tiles, what a step takes by default, both are 256 threads. The LDS is the larger of the two.
 #include "attention_chunk_wg.h"
 #include "attention_decode_wg.h"
 #include "attention_prefill_f32_wg.h"
@@ -49,7 +50,7 @@ __global__ __launch_bounds__(kRaggedThreads) void ragged_kernel(DecodeParams dp,
   }
 }
 
-// The same for chunk rows cut into prefill tiles (16-bit caches): 256-thread
+// The same for chunk rows cut into prefill tiles of a 16-bit cache: 256-thread
 // workgroups of both kinds, two of any per CU. Bound like the prefill kernel
 // in steps with large chunks, by the decode rows' streaming and the tiles'
 // serial chain in small ones. Against the kernel above (us per call): 2 x 512

@@ -271,7 +271,7 @@ __global__ void silu_mul_split_kernel(const T* __restrict__ gu, T* __restrict__ 
 // 23.7 -> 9.9 us (3.9 TB/s), 64 x 151935 72 -> 15, against one piece a thread
 // at a time, or one element where the vocabulary is not a multiple of 4. Four
 // loads, and each row cut over 16 workgroups that exchange (value, index) in the
-// output word, took 24 us.
+// output word, took 22-24 us.
 constexpr int kArgmaxThreads = 1024;
 constexpr int kArgmaxLoads = 8;
 

@@ -16,11 +16,10 @@
 // slice (a prefill chunk) are cut into tiles of chunk_q_tile consecutive
 // positions; each tile's keys 0..last position are cut into partitions of
 // ~chunk_partition_tokens, one ChunkItem each, run on MFMA tiles (16-bit
-// operands with a bf16/fp16 cache, fp32 operands with an fp32 cache). With a
-// 16-bit cache and neither size given, the tiles are prefill tiles instead
-// (cut_prefill below). Split
-// rows of either kind are merged inside their launch by the last partition
-// to finish.
+// operands with a bf16/fp16 cache, fp32 operands with an fp32 cache). With
+// neither size given, and a 16-bit cache or an fp32 one of head_dim 64, the
+// tiles are prefill tiles instead (cut_prefill below). Split rows of either
+// kind are merged inside their launch by the last partition to finish.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -191,7 +190,10 @@ void for_prefill_tiles(const le_step_slice* s, int n, int rows, int bs, F&& f) {
 //   and 31.1; 512 after 1024 35.2, 35.3, 38.0 and 42.8; 4 x 200 after 300, 16/16
 //   heads, 28.5, 28.5, 24.4 and 78).
 // Steps with more rows than arrival counters keep the 32-row tiles: a step
-// that splits nothing there runs without a workspace.
+// that splits nothing there runs without a workspace, and one that does is
+// refused, whichever tiles would run it. (Prefill tiles that stay whole use no
+// counter, so such steps could run on them: 4096 rows and 16 kv heads are the
+// limit, and one decode row more takes the slower tiles.)
 PrefillCut cut_prefill(const le_plan_config& cfg, const le_step_slice* s, int n, int64_t n_tok) {
   PrefillCut c;
   const int group = cfg.q_heads / cfg.kv_heads, bs = cfg.block_size;
