@@ -284,11 +284,6 @@ int ragged_attention(const void* q, le_dtype act_dtype, const void* k_new, const
   const bool two_launches = (cfg.flags & LE_PLAN_TWO_LAUNCHES) != 0;
   if (cfg.chunk_q_tile <= 0) {  // chunk items are prefill tiles
     const bool wide = cfg.chunk_q_tile == le::kWidePrefillTiles;
-    if (whole) {
-      e = le::attention_decode(d, act_dtype, kv_dtype, stream);
-      if (e != hipSuccess) return hip_status(e);
-      return hip_status(le::attention_prefill(c, wide, act_dtype, kv_dtype, stream));
-    }
     return hip_status(plan->n_decode_items > 0
                           ? le::attention_ragged_prefill(d, c, wide, act_dtype, kv_dtype, stream)
                           : le::attention_prefill(c, wide, act_dtype, kv_dtype, stream));

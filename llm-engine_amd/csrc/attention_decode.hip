@@ -43,13 +43,6 @@ __global__ __launch_bounds__(kMfmaThreads) void mfma_kernel_wide(DecodeParams p)
   dec::decode_wg<ACT, KV, HD, kMfmaWaves>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
 }
 
-// The decode rows of a mixed step without a workspace (decode_wg's kWhole).
-template <typename ACT, typename KV, int HD>
-__global__ __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(2))) void mfma_kernel_whole(DecodeParams p) {
-  __shared__ dec::DecodeSmem<KV, HD, kMfmaWaves> sm;
-  dec::decode_wg<ACT, KV, HD, kMfmaWaves, false, true>(p, sm, blockIdx.x, blockIdx.y, blockIdx.z);
-}
-
 // The reference-shaped launch's split rows in a 16-bit cache, with softmax
 // weights in two terms. Longer partitions than nsplit parts of every row leave
 // fewer of a row's heavy weights the largest of theirs (exactly 1): with weights
@@ -73,11 +66,7 @@ hipError_t launch(const DecodeParams& p, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  if (p.items && !p.item_ids) {
-    if (p.k_new) return hipErrorInvalidValue;  // a mixed step has stored its rows
-    if (p.head_dim == 64) mfma_kernel_whole<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);
-    else mfma_kernel_whole<ACT, KV, 128><<<grid, kMfmaThreads, 0, s>>>(p);
-  } else if (p.rms_x && p.rope_max_pos > 0) {
+  if (p.rms_x && p.rope_max_pos > 0) {
     if (p.head_dim == 64) mfma_kernel_fold<ACT, KV, 64><<<grid, kMfmaThreads, 0, s>>>(p);
     else mfma_kernel_fold<ACT, KV, 128><<<grid, kMfmaThreads, 0, s>>>(p);
   } else if (p.head_dim == 64) {

@@ -62,16 +62,18 @@ template <typename KV, int HD> union RaggedPrefillSmem {
   dec::DecodeSmem<KV, HD, pre::kWaves> d;
 };
 
-template <typename ACT, typename KV, int HD, int NC>
+// kWhole: without a workspace, split rows and tiles run whole (instantiations of
+// their own, so that the usual launch is not shaped by it).
+template <typename ACT, typename KV, int HD, int NC, bool kWhole>
 __global__ __launch_bounds__(pre::kThreads, 2) void ragged_prefill_kernel(DecodeParams dp, ChunkParams cp) {
   __shared__ RaggedPrefillSmem<KV, HD> sm;
   const int n_chunk_wg = cp.n_items * cp.kv_heads;
   const int b = blockIdx.x;
   if (b < n_chunk_wg) {
-    pre::prefill_wg<ACT, KV, HD, NC>(cp, sm.c, b / cp.kv_heads, b % cp.kv_heads);
+    pre::prefill_wg<ACT, KV, HD, NC, kWhole>(cp, sm.c, b / cp.kv_heads, b % cp.kv_heads);
   } else {
     const int d = b - n_chunk_wg;
-    dec::decode_wg<ACT, KV, HD, pre::kWaves>(dp, sm.d, d % dp.n_rows, d / dp.n_rows, 0);
+    dec::decode_wg<ACT, KV, HD, pre::kWaves, false, kWhole>(dp, sm.d, d % dp.n_rows, d / dp.n_rows, 0);
   }
 }
 
@@ -83,17 +85,41 @@ template <int HD> union RaggedPrefillF32Smem {
   dec::DecodeSmem<float, HD, pre::kWaves> d;
 };
 
-template <typename ACT, int HD>
+template <typename ACT, int HD, bool kWhole>
 __global__ __launch_bounds__(pre::kThreads, 2) void ragged_prefill_f32_kernel(DecodeParams dp, ChunkParams cp) {
   __shared__ RaggedPrefillF32Smem<HD> sm;
   const int n_chunk_wg = cp.n_items * cp.kv_heads;
   const int b = blockIdx.x;
   if (b < n_chunk_wg) {
-    pre::prefill_f32_wg<ACT, HD>(cp, sm.c, b / cp.kv_heads, b % cp.kv_heads);
+    pre::prefill_f32_wg<ACT, HD, kWhole>(cp, sm.c, b / cp.kv_heads, b % cp.kv_heads);
   } else {
     const int d = b - n_chunk_wg;
-    dec::decode_wg<ACT, float, HD, pre::kWaves>(dp, sm.d, d % dp.n_rows, d / dp.n_rows, 0);
+    dec::decode_wg<ACT, float, HD, pre::kWaves, false, kWhole>(dp, sm.d, d % dp.n_rows, d / dp.n_rows, 0);
   }
+}
+
+}  // namespace
+
+namespace {
+
+template <bool kWhole>
+hipError_t launch_prefill(const DecodeParams& d, const ChunkParams& c, bool wide, int act_dtype, int kv_dtype,
+                          const dim3& grid, hipStream_t s) {
+  return with_dtype(act_dtype, [&](auto a) {
+    if (kv_dtype == LE_F32) {
+      if (c.head_dim != 64 || wide) return hipErrorInvalidValue;
+      ragged_prefill_f32_kernel<decltype(a), 64, kWhole><<<grid, pre::kThreads, 0, s>>>(d, c);
+      return hipGetLastError();
+    }
+    return with_dtype16(kv_dtype, [&](auto k) {
+      using ACT = decltype(a);
+      using KV = decltype(k);
+      if (c.head_dim == 128) ragged_prefill_kernel<ACT, KV, 128, 1, kWhole><<<grid, pre::kThreads, 0, s>>>(d, c);
+      else if (wide) ragged_prefill_kernel<ACT, KV, 64, 2, kWhole><<<grid, pre::kThreads, 0, s>>>(d, c);
+      else ragged_prefill_kernel<ACT, KV, 64, 1, kWhole><<<grid, pre::kThreads, 0, s>>>(d, c);
+      return hipGetLastError();
+    });
+  });
 }
 
 }  // namespace
@@ -103,24 +129,11 @@ hipError_t attention_ragged_prefill(const DecodeParams& d, const ChunkParams& c,
   const int64_t n = static_cast<int64_t>(c.n_items + d.n_rows) * c.kv_heads;
   if (n <= 0) return hipSuccess;
   if (n > 0x7fffffff || d.kv_heads != c.kv_heads || d.head_dim != c.head_dim || !d.items ||
-      (wide && c.head_dim != 64))
+      (d.item_ids == nullptr) != (c.item_ids == nullptr) || (wide && c.head_dim != 64))
     return hipErrorInvalidValue;
   const dim3 grid(static_cast<unsigned>(n));
-  return with_dtype(act_dtype, [&](auto a) {
-    if (kv_dtype == LE_F32) {
-      if (c.head_dim != 64 || wide) return hipErrorInvalidValue;
-      ragged_prefill_f32_kernel<decltype(a), 64><<<grid, pre::kThreads, 0, s>>>(d, c);
-      return hipGetLastError();
-    }
-    return with_dtype16(kv_dtype, [&](auto k) {
-      using ACT = decltype(a);
-      using KV = decltype(k);
-      if (c.head_dim == 128) ragged_prefill_kernel<ACT, KV, 128, 1><<<grid, pre::kThreads, 0, s>>>(d, c);
-      else if (wide) ragged_prefill_kernel<ACT, KV, 64, 2><<<grid, pre::kThreads, 0, s>>>(d, c);
-      else ragged_prefill_kernel<ACT, KV, 64, 1><<<grid, pre::kThreads, 0, s>>>(d, c);
-      return hipGetLastError();
-    });
-  });
+  return d.item_ids ? launch_prefill<false>(d, c, wide, act_dtype, kv_dtype, grid, s)
+                    : launch_prefill<true>(d, c, wide, act_dtype, kv_dtype, grid, s);
 }
 
 hipError_t attention_ragged(const DecodeParams& d, const ChunkParams& c, int act_dtype, int kv_dtype,
